@@ -78,38 +78,64 @@ __device__ __forceinline__ void store_out(float* q, float v) {
     *q = v;
 }
 
-template <int MB, int NB, int EPI, int ACT, bool PRE, bool WT = false>
-__device__ __forceinline__ void epilogue_f32_t(const GemmParams& p, floatx16 (&acc)[MB][NB], const float (&bsum)[NB],
-                                               bool do_bsum, int wm0, int wn0, int split, int lane,
-                                               const float (&auxv)[MB * NB * 16]) {
+// One wave's outputs.  FULL: every row and column is in range (the element
+// loop then has no branch per element, which had the stores of a wave's 64
+// elements one exec-mask change apart).
+template <int MB, int NB, int EPI, int ACT, bool PRE, bool WT, bool FULL>
+__device__ __forceinline__ void epilogue_f32_elems(const GemmParams& p, floatx16 (&acc)[MB][NB], int wm0, int wn0,
+                                                   int split, int lane, const float (&auxv)[MB * NB * 16]) {
   const int h = lane >> 5;
   const int l32 = lane & 31;
   float* C = p.C + (int64_t)split * p.c_split_stride;
 #pragma unroll
   for (int bi = 0; bi < MB; ++bi) {
+    // the activation derivative's inputs of a block row: every load issued
+    // (clamped, not branched around) before the first is used
+    float aux[EPI == EPI_DACT && !PRE ? NB * 16 : 1];
+    if constexpr (EPI == EPI_DACT && !PRE) {
+#pragma unroll
+      for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int gm = wm0 + bi * 32 + 8 * (r >> 2) + 4 * h + (r & 3), gn = wn0 + bj * 32 + l32;
+          aux[16 * bj + r] = p.aux[(int64_t)(FULL ? gm : min(gm, p.M - 1)) * p.ldaux + (FULL ? gn : min(gn, p.N - 1))];
+        }
+    }
 #pragma unroll
     for (int bj = 0; bj < NB; ++bj) {
       const int gn = wn0 + bj * 32 + l32;
-      const bool n_ok = gn < p.N;
+      const bool n_ok = FULL || gn < p.N;
       float bias = 0.f;
       if (EPI == EPI_BIAS_ACT && p.bias && n_ok) bias = PRE ? auxv[bj] : p.bias[gn];
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int gm = wm0 + bi * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (!n_ok || gm >= p.M) continue;
+        if (!FULL && (!n_ok || gm >= p.M)) continue;
         float v = acc[bi][bj][r];
         const int64_t o = (int64_t)gm * p.ldc + gn;
         if (EPI == EPI_BIAS_ACT) {
           v += bias;
           if (p.pre) p.pre[o] = v;
           v = ppo::act_fwd(ACT, v);
-        } else if (EPI == EPI_DACT) {
-          v *= ppo::act_grad(ACT, PRE ? auxv[16 * (bi * NB + bj) + r] : p.aux[(int64_t)gm * p.ldaux + gn]);
+        } else if constexpr (EPI == EPI_DACT) {
+          v *= ppo::act_grad(ACT, PRE ? auxv[16 * (bi * NB + bj) + r] : aux[16 * bj + r]);
         }
         store_out<WT>(C + o, v);
       }
     }
   }
+}
+
+template <int MB, int NB, int EPI, int ACT, bool PRE, bool WT = false>
+__device__ __forceinline__ void epilogue_f32_t(const GemmParams& p, floatx16 (&acc)[MB][NB], const float (&bsum)[NB],
+                                               bool do_bsum, int wm0, int wn0, int split, int lane,
+                                               const float (&auxv)[MB * NB * 16]) {
+  const int h = lane >> 5;
+  const int l32 = lane & 31;
+  if (wm0 + MB * 32 <= p.M && wn0 + NB * 32 <= p.N)
+    epilogue_f32_elems<MB, NB, EPI, ACT, PRE, WT, true>(p, acc, wm0, wn0, split, lane, auxv);
+  else
+    epilogue_f32_elems<MB, NB, EPI, ACT, PRE, WT, false>(p, acc, wm0, wn0, split, lane, auxv);
   if (do_bsum) {
 #pragma unroll
     for (int bj = 0; bj < NB; ++bj) {

@@ -10,12 +10,25 @@
 // 128 x 128 instead of one).  The 8-wave tiles keep three.
 //
 // Tiles: 4 wave64s in 2 x 2 (64 / 128 x 64 / 128 tiles) or 8 in 2 x 4 / 4 x 2
-// (128 x 256, 256 x 128), each wave (BM/WM) x (BN/WN) of 32 x 32 blocks of
-// v_mfma_f32_32x32x2_f32; 32 reduction elements per stage.  The 8-wave tiles
-// read 2-4x fewer operand bytes per FLOP from L2 (a 64 x 64 tile at full fp32
-// MFMA rate needs more L2 bandwidth than the chip has).  Inside each group of
-// 8 reduction elements, lane half h consumes k = 8g + 4h + s at MFMA step s
-// (both operands use the same order, so the sum is unchanged).
+// (128 x 256, 256 x 128), each wave (BM/WM) x (BN/WN) of 32 x 32 blocks; 32
+// reduction elements per stage.  The 8-wave tiles read 2-4x fewer operand
+// bytes per FLOP from L2 (a 64 x 64 tile at full fp32 MFMA rate needs more L2
+// bandwidth than the chip has).  Inside each group of 8 reduction elements,
+// lane half h holds k = 8g + 4h + s (both operands the same order, so the sum
+// is unchanged).
+//
+// Products: v_mfma_f32_32x32x2_f32 for small row-layout problems; else each
+// wave splits the fp32 values it reads from LDS into three bf16 pieces and
+// multiplies those (split_f32.h): six v_mfma_f32_32x32x16_bf16 replace eight
+// fp32 ones at 3/8 of their cycles, and 11 vector instructions per pair of
+// operand values beside them.  With 64 x 64 outputs per wave the matrix cores
+// and the vector unit are about evenly busy (228 TFLOP/s of fp32 products in
+// registers, 151 on fp32 MFMA, 285 without the splitting).  32768 x 256 x 256
+// forward on 256 x 128 tiles 42.6 -> 32-34 us, x 400 with gathered rows 65.7 ->
+// 47, input cotangent 57 -> 41 (tile 2), 256 x 256 x 32768 weight gradient on
+// 64 splits 46 -> 38, 400 x 256 x 32768 on 64 x 64 tiles 83 -> 68.  What is left
+// is the stage barriers and the epilogue of a grid that runs one wave of
+// workgroups.
 // LDS layouts (fp32, 16-byte chunks XOR-swizzled on the copy side):
 //   k-contiguous [ROWS][32]: chunk c of row r at c ^ kc_swizzle(r); an operand
 //     read (4 consecutive k of one row) is one 16-byte read;
@@ -26,6 +39,7 @@
 // by K goes through registers with the elements past K zeroed.
 #include "gemm_f32.h"
 #include "grad_reduce.h"
+#include "split_f32.h"
 
 namespace ppo_f32 {
 namespace {
@@ -137,12 +151,54 @@ __device__ __forceinline__ floatx4 operand(const float* lds, int rbase, int g, i
   }
 }
 
+// A wave's MB x NB blocks from row wm0 and column wn0 over reduction [kb, ke)
+// on v_mfma_f32_32x32x2_f32, operands straight from global memory: the cold
+// path of sums that the split products left not finite.
+template <int MB, int NB, bool A_K, bool B_K>
+__device__ __forceinline__ void exact_wave_tile(const GemmParams& p, floatx16 (&acc)[MB][NB], int wm0, int wn0, int kb,
+                                                int ke, int lane) {
+  const int h = lane >> 5, l32 = lane & 31;
+#pragma unroll
+  for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+    for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[bi][bj][r] = 0.f;
+#pragma unroll 1
+  for (int k0 = kb; k0 < ke; k0 += 2) {
+    const int k = k0 + h;
+    const bool in = k < ke;
+    const int kc = in ? k : kb;
+    float a[MB], b[NB];
+#pragma unroll
+    for (int bi = 0; bi < MB; ++bi) {
+      const int m = min(wm0 + bi * 32 + l32, p.M - 1);
+      const int64_t r = A_K ? m : kc;
+      const int64_t row = p.rows ? (int64_t)p.rows[r] : r;
+      a[bi] = in ? p.A[row * p.lda + (A_K ? kc : m)] : 0.f;
+    }
+#pragma unroll
+    for (int bj = 0; bj < NB; ++bj) {
+      const int n = min(wn0 + bj * 32 + l32, p.N - 1);
+      b[bj] = in ? p.B[B_K ? (int64_t)n * p.ldb + kc : (int64_t)kc * p.ldb + n] : 0.f;
+    }
+#pragma unroll
+    for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < NB; ++bj)
+        acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
+  }
+}
+
 // One BM x BN output tile (tile row tm, column tn) of split `split` of the
 // GEMM p.
 // KIDX: the LDS capacity for a gathered k-outer A's split indices.
 // WT: a weight-gradient store whose partials another workgroup of the launch
 // sums (EPI_STORE only; device-coherent stores).
-template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, int NBUF, int KIDX = F32D_KIDX_MAX, bool WT = false>
+// SPLIT: the products on the bf16 matrix cores (split_f32.h), else
+// v_mfma_f32_32x32x2_f32.
+template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, int NBUF, bool SPLIT, int KIDX = F32D_KIDX_MAX,
+          bool WT = false>
 __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int tn, int split) {
   constexpr int NW = WM * WN;
   constexpr int MB = BM / WM / 32, NB = BN / WN / 32;  // 32 x 32 blocks per wave
@@ -245,31 +301,86 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
     if (kt + NBUF - 1 < nk) issue(kt + NBUF - 1);
     const float* la = sA[kt % NBUF];
     const float* lb = sB[kt % NBUF];
-    floatx4 a4[2][MB], b4[2][NB];
-    auto read_ops = [&](int set, int g) {
+    if constexpr (!SPLIT) {
+      floatx4 a4[2][MB], b4[2][NB];
+      auto read_ops = [&](int set, int g) {
 #pragma unroll
-      for (int bi = 0; bi < MB; ++bi) a4[set][bi] = operand<BM, A_K>(la, wm * (BM / WM) + bi * 32, g, lane);
+        for (int bi = 0; bi < MB; ++bi) a4[set][bi] = operand<BM, A_K>(la, wm * (BM / WM) + bi * 32, g, lane);
 #pragma unroll
-      for (int bj = 0; bj < NB; ++bj) b4[set][bj] = operand<BN, B_K>(lb, wn * (BN / WN) + bj * 32, g, lane);
-    };
-    read_ops(0, 0);
+        for (int bj = 0; bj < NB; ++bj) b4[set][bj] = operand<BN, B_K>(lb, wn * (BN / WN) + bj * 32, g, lane);
+      };
+      read_ops(0, 0);
 #pragma unroll
-    for (int g = 0; g < BK / 8; ++g) {
-      const int cur = g & 1;
-      if (g + 1 < BK / 8) read_ops(cur ^ 1, g + 1);
+      for (int g = 0; g < BK / 8; ++g) {
+        const int cur = g & 1;
+        if (g + 1 < BK / 8) read_ops(cur ^ 1, g + 1);
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+        for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int bi = 0; bi < MB; ++bi)
+          for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < NB; ++bj)
+              acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[cur][bi][s], b4[cur][bj][s], acc[bi][bj], 0, 0, 0);
+        if (do_bsum) {
 #pragma unroll
           for (int bj = 0; bj < NB; ++bj)
-            acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[cur][bi][s], b4[cur][bj][s], acc[bi][bj], 0, 0, 0);
-      if (do_bsum) {
+            bsum[bj] += (b4[cur][bj][0] + b4[cur][bj][1]) + (b4[cur][bj][2] + b4[cur][bj][3]);
+        }
+      }
+    } else {
+      // a 16-deep block of the reduction (two groups per lane half), the next
+      // block's LDS reads issued before this block's products
+      floatx4 a4[2][2][MB], b4[2][2][NB];
+      auto read_ops = [&](int set, int blk) {
 #pragma unroll
-        for (int bj = 0; bj < NB; ++bj)
-          bsum[bj] += (b4[cur][bj][0] + b4[cur][bj][1]) + (b4[cur][bj][2] + b4[cur][bj][3]);
+        for (int q = 0; q < 2; ++q) {
+#pragma unroll
+          for (int bi = 0; bi < MB; ++bi)
+            a4[set][q][bi] = operand<BM, A_K>(la, wm * (BM / WM) + bi * 32, 2 * blk + q, lane);
+#pragma unroll
+          for (int bj = 0; bj < NB; ++bj)
+            b4[set][q][bj] = operand<BN, B_K>(lb, wn * (BN / WN) + bj * 32, 2 * blk + q, lane);
+        }
+      };
+      read_ops(0, 0);
+#pragma unroll
+      for (int blk = 0; blk < BK / 16; ++blk) {
+        const int cur = blk & 1;
+        if (blk + 1 < BK / 16) read_ops(cur ^ 1, blk + 1);
+        ppo::Split8 fa[MB], fb[NB];
+#pragma unroll
+        for (int bi = 0; bi < MB; ++bi) fa[bi] = ppo::split8(a4[cur][0][bi], a4[cur][1][bi]);
+#pragma unroll
+        for (int bj = 0; bj < NB; ++bj) fb[bj] = ppo::split8(b4[cur][0][bj], b4[cur][1][bj]);
+#pragma unroll
+        for (int t = 0; t < ppo::SPLIT_PRODUCTS; ++t)
+#pragma unroll
+          for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < NB; ++bj) acc[bi][bj] = ppo::split_mfma(t, fa[bi], fb[bj], acc[bi][bj]);
+        if (do_bsum) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int bj = 0; bj < NB; ++bj)
+              bsum[bj] += (b4[cur][q][bj][0] + b4[cur][q][bj][1]) + (b4[cur][q][bj][2] + b4[cur][q][bj][3]);
+        }
       }
     }
+  }
+
+  if constexpr (SPLIT) {
+    // an infinity (or a value that rounds to one in bf16) has no finite split:
+    // a wave whose sums are not all finite forms them again on fp32 MFMA
+    float nonfinite = 0.f;
+#pragma unroll
+    for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+      for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) nonfinite = __fmaf_rn(acc[bi][bj][r], 0.f, nonfinite);
+    if (__builtin_expect(__any(nonfinite != 0.f), 0))
+      exact_wave_tile<MB, NB, A_K, B_K>(p, acc, m0 + wm * (BM / WM), n0 + wn * (BN / WN), kb, ke, lane);
   }
 
   if constexpr (WT)
@@ -281,12 +392,12 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
     epilogue_f32<MB, NB>(p, acc, bsum, do_bsum, m0 + wm * (BM / WM), n0 + wn * (BN / WN), split, lane, auxv);
 }
 
-template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, int NBUF>
-__global__ void __launch_bounds__(WM * WN * 64) gemm_f32d_kernel(GemmParams p0) {
+template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, int NBUF, bool SPLIT>
+__global__ void __launch_bounds__(WM * WN * 64, 2) gemm_f32d_kernel(GemmParams p0) {
   const ppo::TileCoord tc = ppo::xcd_tile();
   const int tower = tc.z / p0.splits;
   const int split = tc.z - tower * p0.splits;
-  gemm_f32d_tile<BM, BN, WM, WN, A_K, B_K, NBUF>(tower_params(p0, tower), tc.m, tc.n, split);
+  gemm_f32d_tile<BM, BN, WM, WN, A_K, B_K, NBUF, SPLIT>(tower_params(p0, tower), tc.m, tc.n, split);
 }
 
 // Several GEMMs of one tile shape in one launch: problem i owns the linear
@@ -303,7 +414,7 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32d_group_kernel(F32Group 
   int i = 0;
   while (i + 1 < g.count && t >= g.start[i + 1]) ++i;
   const int local = t - g.start[i];
-  gemm_f32d_tile<BM, BN, WM, WN, A_K, B_K, NBUF>(g.p[i], (local / g.gx[i]) % g.gy[i], local % g.gx[i],
+  gemm_f32d_tile<BM, BN, WM, WN, A_K, B_K, NBUF, true>(g.p[i], (local / g.gx[i]) % g.gy[i], local % g.gx[i],
                                                  local / (g.gx[i] * g.gy[i]));
 }
 
@@ -337,7 +448,7 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32d_group_final_kernel(F32
   const GemmParams& p = g.p[i];
   const int local = t - g.start[i];
   const int tm = (local / g.gx[i]) % g.gy[i], tn = local % g.gx[i];
-  gemm_f32d_tile<BM, BN, WM, WN, false, false, NBUF, KIDX, true>(p, tm, tn, local / (g.gx[i] * g.gy[i]));
+  gemm_f32d_tile<BM, BN, WM, WN, false, false, NBUF, true, KIDX, true>(p, tm, tn, local / (g.gx[i] * g.gy[i]));
   // every wave's partial stores complete, then one arrival for the tile
   const int slot = f.slot0[i] + tm * g.gx[i] + tn;
   double sq = 0.0;
@@ -373,23 +484,42 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32d_group_final_kernel(F32
   ppo_gr::block_sumsq<WM * WN * 64>(sq, s_w, f.sumsq + slot);
 }
 
-template <int BM, int BN, int WM, int WN, bool A_K, bool B_K>
+template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, bool SPLIT = true>
 int launch(hipStream_t st, const GemmParams& p, int splits) {
   constexpr int NBUF = WM * WN == 4 ? 2 : 3;
   dim3 grid(ppo::ceil_div(p.N, BN), ppo::ceil_div(p.M, BM), splits * p.towers);
-  hipLaunchKernelGGL((gemm_f32d_kernel<BM, BN, WM, WN, A_K, B_K, NBUF>), grid, dim3(WM * WN * 64), 0, st, p);
+  hipLaunchKernelGGL((gemm_f32d_kernel<BM, BN, WM, WN, A_K, B_K, NBUF, SPLIT>), grid, dim3(WM * WN * 64), 0, st, p);
   return ppo::check_launch("ppo_gemm_f32");
+}
+
+// Whether a problem's products run on the bf16 matrix cores.  Weight
+// gradients always; the row layouts from 2^21 outputs on: there the matrix
+// cores bound the launch (32768 x 256 x 256 forward on 64 x 64 tiles 45.7 ->
+// 39.4 us, 4096 x 512 x 512 27.5 -> 24.6), below it latency does and the
+// splitting's vector work is in the way (2048 x 256 x 256 x two towers 13.2
+// -> 13.6 us, 1024 x 768 x 256 10.1 -> 10.1).  By the problem's size
+// alone, so every tile of one problem forms the same bits (tiles 1, 2, 8 and
+// 9, which only large problems take, are compiled split).
+template <bool A_K>
+bool split_products(const GemmParams& p) {
+  return !A_K || (int64_t)p.M * p.N >= (1 << 21);
 }
 
 template <bool A_K, bool B_K>
 int launch_tile(hipStream_t st, const GemmParams& p, int splits, int tile) {
   switch (tile) {
-    case 0: return launch<128, 128, 2, 2, A_K, B_K>(st, p, splits);
+    case 0:
+      if constexpr (A_K)
+        if (!split_products<A_K>(p)) return launch<128, 128, 2, 2, A_K, B_K, false>(st, p, splits);
+      return launch<128, 128, 2, 2, A_K, B_K>(st, p, splits);
     case 1: return launch<128, 64, 2, 2, A_K, B_K>(st, p, splits);
     case 2: return launch<64, 128, 2, 2, A_K, B_K>(st, p, splits);
     case 8: return launch<128, 256, 2, 4, A_K, B_K>(st, p, splits);
     case 9: return launch<256, 128, 4, 2, A_K, B_K>(st, p, splits);
-    default: return launch<64, 64, 2, 2, A_K, B_K>(st, p, splits);
+    default:
+      if constexpr (A_K)
+        if (!split_products<A_K>(p)) return launch<64, 64, 2, 2, A_K, B_K, false>(st, p, splits);
+      return launch<64, 64, 2, 2, A_K, B_K>(st, p, splits);
   }
 }
 

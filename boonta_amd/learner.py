@@ -393,19 +393,20 @@ class ForwardChain:
 
     @staticmethod
     def _f32_tile(a_layout: int, b_layout: int, M: int, K: int) -> int:
-        """fp32 tile for a whole-minibatch contraction, measured per update:
-        over 32768 rows or more (the Anakin minibatch) the 8-wave 256 x 128
-        tile for forwards and 128 x 128 for the weight gradient of a 256-row
-        kernel (11.43 -> 11.31 ms per update); at 16384 rows (the GRU
-        workload) both were slower (17.8 -> 28.2 us on 16384 x 256 x 128,
-        76 -> 90 us on its 256 x 768 dW), so below that the library's default
-        (64 x 64).  The input cotangent (B = W^T) of a 32768-row minibatch
-        also stays on 64 x 64: 10.18 ms per Anakin update against 10.54
-        (256 x 128), 10.47 (128 x 128) and 10.51 (128 x 256)."""
+        """fp32 tile for a whole-minibatch contraction (every tile of one
+        problem forms the same bits).  From 32768 rows (the Anakin minibatch)
+        the 8-wave 256 x 128 tile for forwards (32768 x 256 x 400: 47 us, 61 on
+        64 x 64) and 64 x 128 for the weight gradient of a 256-row kernel (38
+        us against 42; 128 x 128 the same); from 16384 rows 64 x 128 for the
+        input cotangents (B = W^T; 32768 x 256 x 256: 41 us against 44,
+        16384 x 256 x 768: 52 against 61).  Smaller minibatches and every other
+        shape: the library's default 64 x 64, whose grid fills more CUs."""
         if a_layout == A_ROW and b_layout == B_KN and M >= 32768:
             return 9
+        if a_layout == A_ROW and b_layout == B_NK and M >= 16384:
+            return 2
         if a_layout == A_COL and M == 256 and K >= 32768:
-            return 0
+            return 2
         return -1
 
     def _gemm(self, st, a_layout, b_layout, A, lda, rows, B, ldb, C, ldc, M, N, K, splits, stride, epi, bias, act,
