@@ -22,14 +22,14 @@
 // Layout and parallelism: element (n, t, f) at (n * steps + t) * features + f.
 // Each lane owns VW = 4 consecutive features of one sequence where the rows
 // allow (one 16-byte float32 or 8-byte bf16 access), so every step reads one
-// coalesced row.  When the
-// batch x feature lanes alone cannot fill the chip, the time axis is cut into
-// C <= 16 chunks, one wave each, in one workgroup: every wave first folds its
-// chunk into the affine map (A, B) of h_end = A h_start + B, the waves
-// exchange the maps through LDS, and each wave composes the maps before it (in
-// time order for the forward, in reverse for the backward) to start its own
-// chunk from the exact carry, then re-reads the chunk and writes its outputs.
-#include "common.h"
+// coalesced row.  The time axis is cut into chunks of a few steps, one wave
+// each: a wave loads its chunk into registers, folds it into the affine map
+// (A, B) of h_end = A h_start + B, the waves exchange the maps through LDS, and
+// each composes the maps before it (in time order for the forward, in reverse
+// for the backward) to write its chunk's outputs from the exact carry.
+// Sequences of up to 128 steps are one such tile of 16 chunks, longer ones run
+// tile after tile.
+#include "split_f32.h"
 
 #include <algorithm>
 
@@ -58,18 +58,22 @@ __device__ __forceinline__ void store_vec(float* p, int64_t i, const float (&v)[
   x[0] = v[0]; x[1] = v[1]; x[2] = v[2]; x[3] = v[3];
   *reinterpret_cast<floatx4*>(p + i) = x;
 }
+// (rounded by v_cvt_pk_bf16_f32, two values an instruction: to nearest even,
+// as ppo::bf16_bits rounds in nine)
 __device__ __forceinline__ void store_vec(uint16_t* p, int64_t i, const float (&v)[1]) {
-  p[i] = (uint16_t)ppo::bf16_bits(v[0]);
+  p[i] = (uint16_t)ppo::pack_bf16(v[0], v[0]);
 }
 __device__ __forceinline__ void store_vec(uint16_t* p, int64_t i, const float (&v)[4]) {
   uint2 x;
-  x.x = ppo::bf16_bits(v[0]) | (ppo::bf16_bits(v[1]) << 16);
-  x.y = ppo::bf16_bits(v[2]) | (ppo::bf16_bits(v[3]) << 16);
+  x.x = ppo::pack_bf16(v[0], v[1]);
+  x.y = ppo::pack_bf16(v[2], v[3]);
   *reinterpret_cast<uint2*>(p + i) = x;
 }
 // The value a stored element of type S holds (identity for float32).
 __device__ __forceinline__ float stored(float x, const float*) { return x; }
-__device__ __forceinline__ float stored(float x, const uint16_t*) { return ppo::bf16_round(x); }
+__device__ __forceinline__ float stored(float x, const uint16_t*) {
+  return __uint_as_float(ppo::pack_bf16(x, x) << 16);
+}
 
 struct ScanArgs {
   const void* a;
@@ -79,7 +83,7 @@ struct ScanArgs {
   void* out;         // forward: h; backward: db
   void* da;
   void* dinit;
-  int steps, F, chunk;
+  int steps, F;
   const uint8_t* done;  // [batch, steps] episode starts of the SSM block, or null
   const void* reset;    // [batch, features] carry a done step restarts from, or null (zeros)
 };
@@ -140,170 +144,6 @@ __device__ __forceinline__ void reset_da(const ScanArgs& p, const S* a, int64_t 
 #pragma unroll
     for (int k = 0; k < VW; ++k) dav[k] = stored(rv[k] * dv[k], a);
   }
-}
-
-template <typename S, int VW>
-__global__ void __launch_bounds__(64 * MAX_CHUNKS) scan_fwd_kernel(ScanArgs p) {
-  // per chunk: the (A, B) maps of its 64 x VW lanes (dynamic: none when C = 1)
-  extern __shared__ float smem[];
-  float* sA = smem;
-  float* sB = smem + (blockDim.x >> 6) * 64 * VW;
-  const S* a = static_cast<const S*>(p.a);
-  const S* b = static_cast<const S*>(p.b);
-  const S* init = static_cast<const S*>(p.init);
-  S* out = static_cast<S*>(p.out);
-  const int lane = threadIdx.x & 63, c = threadIdx.x >> 6, C = blockDim.x >> 6;
-  const int f0 = (blockIdx.x * 64 + lane) * VW;
-  const bool ok = f0 < p.F;
-  const int64_t n = blockIdx.y;
-  const int t0 = c * p.chunk, t1 = min(p.steps, t0 + p.chunk);
-  const int64_t base = n * (int64_t)p.steps * p.F + f0;
-  float h[VW];
-  if (ok) {
-    load_vec(init, n * (int64_t)p.F + f0, h);
-  } else {
-#pragma unroll
-    for (int k = 0; k < VW; ++k) h[k] = 0.f;
-  }
-  if (C > 1) {
-    float A[VW], B[VW];
-#pragma unroll
-    for (int k = 0; k < VW; ++k) { A[k] = 1.f; B[k] = 0.f; }
-    if (ok) {
-#pragma unroll 4
-      for (int t = t0; t < t1; ++t) {
-        float av[VW], bv[VW];
-        load_ab<S, VW>(p, a, b, base, n, t, f0, av, bv);
-#pragma unroll
-        for (int k = 0; k < VW; ++k) {
-          A[k] = av[k] * A[k];
-          B[k] = av[k] * B[k] + bv[k];
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < VW; ++k) {
-      sA[(c * 64 + lane) * VW + k] = A[k];
-      sB[(c * 64 + lane) * VW + k] = B[k];
-    }
-    __syncthreads();
-    for (int cc = 0; cc < c; ++cc) {
-#pragma unroll
-      for (int k = 0; k < VW; ++k) h[k] = sA[(cc * 64 + lane) * VW + k] * h[k] + sB[(cc * 64 + lane) * VW + k];
-    }
-  }
-  if (!ok) return;
-#pragma unroll 8
-  for (int t = t0; t < t1; ++t) {
-    float av[VW], bv[VW];
-    load_ab<S, VW>(p, a, b, base, n, t, f0, av, bv);
-#pragma unroll
-    for (int k = 0; k < VW; ++k) h[k] = av[k] * h[k] + bv[k];
-    store_vec(out, base + (int64_t)t * p.F, h);
-  }
-}
-
-template <typename S, int VW>
-__global__ void __launch_bounds__(64 * MAX_CHUNKS) scan_bwd_kernel(ScanArgs p) {
-  extern __shared__ float smem[];
-  float* sA = smem;
-  float* sB = smem + (blockDim.x >> 6) * 64 * VW;
-  const S* a = static_cast<const S*>(p.a);
-  const S* g = static_cast<const S*>(p.b);
-  const S* hs = static_cast<const S*>(p.h);
-  const S* init = static_cast<const S*>(p.init);
-  S* db = static_cast<S*>(p.out);
-  S* da = static_cast<S*>(p.da);
-  S* dinit = static_cast<S*>(p.dinit);
-  const int lane = threadIdx.x & 63, c = threadIdx.x >> 6, C = blockDim.x >> 6;
-  const int f0 = (blockIdx.x * 64 + lane) * VW;
-  const bool ok = f0 < p.F;
-  const int64_t n = blockIdx.y;
-  const int t0 = c * p.chunk, t1 = min(p.steps, t0 + p.chunk);
-  const int64_t base = n * (int64_t)p.steps * p.F + f0;
-  // reverse recurrence d_t = g_t + alpha_t d_{t+1}, alpha_t = a_{t+1}
-  // (0 past the last step); d entering this chunk from the chunks after it
-  float d[VW];
-#pragma unroll
-  for (int k = 0; k < VW; ++k) d[k] = 0.f;
-  if (C > 1) {
-    float P[VW], Q[VW];
-#pragma unroll
-    for (int k = 0; k < VW; ++k) { P[k] = 1.f; Q[k] = 0.f; }
-    if (ok) {
-#pragma unroll 4
-      for (int t = t1 - 1; t >= t0; --t) {
-        float al[VW], gv[VW];
-        load_alpha<S, VW>(p, a, base, n, t, al);
-        load_vec(g, base + (int64_t)t * p.F, gv);
-#pragma unroll
-        for (int k = 0; k < VW; ++k) {
-          P[k] = al[k] * P[k];
-          Q[k] = al[k] * Q[k] + gv[k];
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < VW; ++k) {
-      sA[(c * 64 + lane) * VW + k] = P[k];
-      sB[(c * 64 + lane) * VW + k] = Q[k];
-    }
-    __syncthreads();
-    for (int cc = C - 1; cc > c; --cc) {
-#pragma unroll
-      for (int k = 0; k < VW; ++k) d[k] = sA[(cc * 64 + lane) * VW + k] * d[k] + sB[(cc * 64 + lane) * VW + k];
-    }
-  }
-  if (!ok) return;
-  // one step of the reverse recurrence; has_next: a_{t+1} exists; first: t = 0
-  // (h_{t-1} is init, and dinit is written)
-  auto step = [&](int t, bool has_next, bool first) {
-    float al[VW], gv[VW], hp[VW];
-    if (has_next) {
-      load_alpha<S, VW>(p, a, base, n, t, al);
-    } else {
-#pragma unroll
-      for (int k = 0; k < VW; ++k) al[k] = 0.f;
-    }
-    load_vec(g, base + (int64_t)t * p.F, gv);
-    if (first) {
-      load_vec(init, n * (int64_t)p.F + f0, hp);
-    } else {
-      load_vec(hs, base + (int64_t)(t - 1) * p.F, hp);
-    }
-    float dv[VW], dav[VW];
-#pragma unroll
-    for (int k = 0; k < VW; ++k) {
-      d[k] = al[k] * d[k] + gv[k];
-      dv[k] = stored(d[k], db);
-      dav[k] = dv[k] * hp[k];
-    }
-    reset_da<S, VW>(p, a, n, t, f0, dv, dav);
-    store_vec(db, base + (int64_t)t * p.F, d);
-    store_vec(da, base + (int64_t)t * p.F, dav);
-    if (first) {
-      float a0[VW], di[VW];
-      load_vec(a, base, a0);
-      if (is_done(p, n, 0)) {
-#pragma unroll
-        for (int k = 0; k < VW; ++k) a0[k] = 0.f;
-      }
-#pragma unroll
-      for (int k = 0; k < VW; ++k) di[k] = dv[k] * a0[k];
-      store_vec(dinit, n * (int64_t)p.F + f0, di);
-    }
-  };
-  // the last and the first step peeled, so the main loop is branch-free and
-  // its loads can run ahead of the dependent multiply-adds
-  int t = t1 - 1;
-  if (t == p.steps - 1) {
-    step(t, false, t == 0);
-    --t;
-  }
-  const int lo = max(t0, 1);
-#pragma unroll 8
-  for (; t >= lo; --t) step(t, true, false);
-  if (t == 0 && t >= t0) step(0, true, true);
 }
 
 // Register-resident chunks: each wave loads its chunk of at most RL steps once
@@ -469,19 +309,265 @@ __global__ void __launch_bounds__(64 * MAX_CHUNKS) scan_bwd_reg_kernel(ScanArgs 
   }
 }
 
+// Long sequences: the workgroup's waves take the register-resident chunks of
+// one tile of steps after another, the state entering a tile carried in
+// registers from the tile before it, and the next tile's loads issued before
+// this tile's maps are exchanged.  Every operand is read once.  What bounds it
+// is HBM: [128, 1000, 512] bf16 with resets, forward 153 -> 78 us, backward 296
+// -> 130 us, 5.0 TB/s (chunks that re-read their operands before).  A
+// chunk holds 8 steps of operands and the next 8 in storage type, so a
+// workgroup has 8 waves (16 of them spilled registers).
+constexpr int TILE_WAVES = 8;
+
+template <typename S, int VW> struct Raw;
+template <> struct Raw<float, 4> { floatx4 v; };
+template <> struct Raw<float, 1> { float v; };
+template <> struct Raw<uint16_t, 4> { uint2 v; };
+template <> struct Raw<uint16_t, 1> { uint16_t v; };
+
+template <typename S, int VW>
+__device__ __forceinline__ Raw<S, VW> load_raw(const S* p, int64_t i) {
+  return Raw<S, VW>{*reinterpret_cast<const decltype(Raw<S, VW>::v)*>(p + i)};
+}
+__device__ __forceinline__ void expand(const Raw<float, 4>& r, float (&v)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = r.v[k];
+}
+__device__ __forceinline__ void expand(const Raw<float, 1>& r, float (&v)[1]) { v[0] = r.v; }
+__device__ __forceinline__ void expand(const Raw<uint16_t, 4>& r, float (&v)[4]) {
+  v[0] = __uint_as_float(r.v.x << 16); v[1] = __uint_as_float(r.v.x & 0xffff0000u);
+  v[2] = __uint_as_float(r.v.y << 16); v[3] = __uint_as_float(r.v.y & 0xffff0000u);
+}
+__device__ __forceinline__ void expand(const Raw<uint16_t, 1>& r, float (&v)[1]) { v[0] = bf16_to_f32(r.v); }
+
+// Every wave's LDS writes so far are visible to the workgroup; loads from
+// global memory stay in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Bit i: step t0 + i (below steps) of sequence n restarts.
+__device__ __forceinline__ uint32_t done_bits(uint8_t flag, bool live) { return (uint32_t)__ballot(live && flag); }
+
+template <typename S, int VW>
+__global__ void __launch_bounds__(64 * TILE_WAVES) scan_fwd_tile_kernel(ScanArgs p) {
+  __shared__ float sA[2][TILE_WAVES * 64 * VW], sB[2][TILE_WAVES * 64 * VW];
+  const S* a = static_cast<const S*>(p.a);
+  const S* b = static_cast<const S*>(p.b);
+  S* out = static_cast<S*>(p.out);
+  const int lane = threadIdx.x & 63;
+  constexpr int C = TILE_WAVES, TL = RL;
+  const int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int f0 = (blockIdx.x * 64 + lane) * VW;
+  const bool ok = f0 < p.F;
+  const int64_t n = blockIdx.y;
+  const int fc = ok ? f0 : 0;  // lanes past the row read its start and store nothing
+  const int64_t base = n * (int64_t)p.steps * p.F + fc;
+  float h[VW], rv[VW];
+  load_vec(static_cast<const S*>(p.init), n * (int64_t)p.F + fc, h);
+  load_reset<S, VW>(p, n, fc, rv);
+  Raw<S, VW> ra[2][TL], rb[2][TL];
+  uint8_t rd[2] = {0, 0};
+  auto fetch = [&](int set, int t0) {
+#pragma unroll
+    for (int i = 0; i < TL; ++i) {
+      const int64_t o = base + (int64_t)min(t0 + i, p.steps - 1) * p.F;
+      ra[set][i] = load_raw<S, VW>(a, o);
+      rb[set][i] = load_raw<S, VW>(b, o);
+    }
+    if (p.done) rd[set] = p.done[n * p.steps + min(t0 + min(lane, TL - 1), p.steps - 1)];
+  };
+  const int tile = C * TL;
+  auto step_tile = [&](int set, int t0) {
+    // the chunk's operands (the identity map past the last step)
+    const uint32_t done = p.done ? done_bits(rd[set], lane < TL) : 0u;
+    float av[TL][VW], bv[TL][VW], A[VW], B[VW];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) { A[k] = 1.f; B[k] = 0.f; }
+#pragma unroll
+    for (int i = 0; i < TL; ++i) {
+      expand(ra[set][i], av[i]);
+      expand(rb[set][i], bv[i]);
+      const bool live = t0 + i < p.steps;
+#pragma unroll
+      for (int k = 0; k < VW; ++k) {
+        bv[i][k] = live ? bv[i][k] : 0.f;
+        av[i][k] = live ? av[i][k] : 1.f;
+      }
+    }
+    if (done) {  // a restart in this chunk
+#pragma unroll
+      for (int i = 0; i < TL; ++i) {
+        if (!((done >> i) & 1) || t0 + i >= p.steps) continue;
+#pragma unroll
+        for (int k = 0; k < VW; ++k) {
+          bv[i][k] = stored(bv[i][k] + stored(av[i][k] * rv[k], a), a);
+          av[i][k] = 0.f;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TL; ++i) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) {
+        A[k] = av[i][k] * A[k];
+        B[k] = av[i][k] * B[k] + bv[i][k];
+      }
+    }
+    float* pa = sA[set];
+    float* pb = sB[set];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) {
+      pa[(c * 64 + lane) * VW + k] = A[k];
+      pb[(c * 64 + lane) * VW + k] = B[k];
+    }
+    if (t0 - c * TL + tile < p.steps) fetch(set ^ 1, t0 + tile);
+    lds_barrier();
+    float hc[VW];
+#pragma unroll
+    for (int cc = 0; cc < C; ++cc) {
+      if (cc == c) {
+#pragma unroll
+        for (int k = 0; k < VW; ++k) hc[k] = h[k];
+      }
+#pragma unroll
+      for (int k = 0; k < VW; ++k) h[k] = pa[(cc * 64 + lane) * VW + k] * h[k] + pb[(cc * 64 + lane) * VW + k];
+    }
+#pragma unroll
+    for (int i = 0; i < TL; ++i) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) hc[k] = av[i][k] * hc[k] + bv[i][k];
+      if (ok && t0 + i < p.steps) store_vec(out, base + (int64_t)(t0 + i) * p.F, hc);
+    }
+  };
+  fetch(0, c * TL);
+  // (the register sets alternate by unrolling, so that each is indexed by a constant)
+  for (int t0 = c * TL, done_steps = 0; done_steps < p.steps; done_steps += 2 * tile, t0 += 2 * tile) {
+    step_tile(0, t0);
+    if (done_steps + tile < p.steps) step_tile(1, t0 + tile);
+  }
+}
+
+template <typename S, int VW>
+__global__ void __launch_bounds__(64 * TILE_WAVES) scan_bwd_tile_kernel(ScanArgs p) {
+  __shared__ float sA[2][TILE_WAVES * 64 * VW], sB[2][TILE_WAVES * 64 * VW];
+  const S* a = static_cast<const S*>(p.a);
+  const S* g = static_cast<const S*>(p.b);
+  const S* hs = static_cast<const S*>(p.h);
+  const S* init = static_cast<const S*>(p.init);
+  S* db = static_cast<S*>(p.out);
+  S* da = static_cast<S*>(p.da);
+  S* dinit = static_cast<S*>(p.dinit);
+  const int lane = threadIdx.x & 63;
+  constexpr int C = TILE_WAVES, TL = sizeof(S) * VW > 8 ? 4 : RL;  // 8 float4 steps spill
+  const int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int f0 = (blockIdx.x * 64 + lane) * VW;
+  const bool ok = f0 < p.F;
+  const int64_t n = blockIdx.y;
+  const int fc = ok ? f0 : 0;
+  const int64_t base = n * (int64_t)p.steps * p.F + fc;
+  float d[VW], rv[VW];
+#pragma unroll
+  for (int k = 0; k < VW; ++k) d[k] = 0.f;
+  load_reset<S, VW>(p, n, fc, rv);
+  // of step t: a_{t+1}, g_t, h_{t-1} (init at t = 0); the flags of steps t0 .. t0 + TL
+  Raw<S, VW> ra[2][TL], rg[2][TL], rh[2][TL];
+  uint8_t rd[2] = {0, 0};
+  auto fetch = [&](int set, int t0) {
+#pragma unroll
+    for (int i = 0; i < TL; ++i) {
+      const int t = min(t0 + i, p.steps - 1);
+      ra[set][i] = load_raw<S, VW>(a, base + (int64_t)min(t + 1, p.steps - 1) * p.F);
+      rg[set][i] = load_raw<S, VW>(g, base + (int64_t)t * p.F);
+      rh[set][i] = load_raw<S, VW>(t > 0 ? hs : init, t > 0 ? base + (int64_t)(t - 1) * p.F : n * (int64_t)p.F + fc);
+    }
+    if (p.done) rd[set] = p.done[n * p.steps + min(t0 + min(lane, TL), p.steps - 1)];
+  };
+  const int tile = C * TL;
+  const int ntiles = (p.steps + tile - 1) / tile;
+  auto step_tile = [&](int set, int it) {
+    const int t0 = it * tile + c * TL;
+    const uint32_t done = p.done ? done_bits(rd[set], lane <= TL) : 0u;
+    float al[TL][VW], gv[TL][VW], hp[TL][VW], P[VW], Q[VW];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) { P[k] = 1.f; Q[k] = 0.f; }
+#pragma unroll
+    for (int i = TL - 1; i >= 0; --i) {
+      expand(ra[set][i], al[i]);
+      expand(rg[set][i], gv[i]);
+      expand(rh[set][i], hp[i]);
+      // no decay into a restarted step or past the last one; the identity past the end
+      const bool live = t0 + i < p.steps, cut = t0 + i + 1 >= p.steps || ((done >> (i + 1)) & 1);
+#pragma unroll
+      for (int k = 0; k < VW; ++k) {
+        al[i][k] = live ? (cut ? 0.f : al[i][k]) : 1.f;
+        gv[i][k] = live ? gv[i][k] : 0.f;
+        P[k] = al[i][k] * P[k];
+        Q[k] = al[i][k] * Q[k] + gv[i][k];
+      }
+    }
+    float* pa = sA[set];
+    float* pb = sB[set];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) {
+      pa[(c * 64 + lane) * VW + k] = P[k];
+      pb[(c * 64 + lane) * VW + k] = Q[k];
+    }
+    if (it > 0) fetch(set ^ 1, t0 - tile);
+    lds_barrier();
+    float dc[VW];
+#pragma unroll
+    for (int cc = C - 1; cc >= 0; --cc) {
+      if (cc == c) {
+#pragma unroll
+        for (int k = 0; k < VW; ++k) dc[k] = d[k];
+      }
+#pragma unroll
+      for (int k = 0; k < VW; ++k) d[k] = pa[(cc * 64 + lane) * VW + k] * d[k] + pb[(cc * 64 + lane) * VW + k];
+    }
+#pragma unroll
+    for (int i = TL - 1; i >= 0; --i) {
+      const int t = t0 + i;
+      float dv[VW], dav[VW];
+#pragma unroll
+      for (int k = 0; k < VW; ++k) {
+        dc[k] = al[i][k] * dc[k] + gv[i][k];
+        dv[k] = stored(dc[k], db);
+        dav[k] = dv[k] * hp[i][k];
+      }
+      if ((done >> i) & 1) {
+#pragma unroll
+        for (int k = 0; k < VW; ++k) dav[k] = stored(rv[k] * dv[k], a);
+      }
+      if (ok && t < p.steps) {
+        store_vec(db, base + (int64_t)t * p.F, dc);
+        store_vec(da, base + (int64_t)t * p.F, dav);
+        if (t == 0) {
+          float a0[VW], di[VW];
+          load_vec(a, base, a0);
+#pragma unroll
+          for (int k = 0; k < VW; ++k) di[k] = dv[k] * ((done & 1) ? 0.f : a0[k]);
+          store_vec(dinit, n * (int64_t)p.F + f0, di);
+        }
+      }
+    }
+  };
+  int it = ntiles - 1;
+  fetch(0, it * tile + c * TL);
+  for (; it >= 0; it -= 2) {
+    step_tile(0, it);
+    if (it > 0) step_tile(1, it - 1);
+  }
+}
+
 bool aligned(const void* ptr, int bytes) { return (reinterpret_cast<uintptr_t>(ptr) % bytes) == 0; }
 
 template <typename S, int VW, bool BWD>
-int launch(hipStream_t st, const ScanArgs& p, int batch) {
-  const int lanes = ppo::ceil_div(p.F, VW);
-  const int groups = ppo::ceil_div(lanes, 64);
-  const int C = ppo::ceil_div(p.steps, p.chunk);
-  dim3 grid(groups, batch), block(64 * C);
-  const size_t lds = C > 1 ? 2 * sizeof(float) * (size_t)C * 64 * VW : 0;
-  if (BWD) {
-    hipLaunchKernelGGL((scan_bwd_kernel<S, VW>), grid, block, lds, st, p);
+int launch_tile(hipStream_t st, const ScanArgs& p, int batch) {
+  const int groups = ppo::ceil_div(ppo::ceil_div(p.F, VW), 64);
+  dim3 grid(groups, batch), block(64 * TILE_WAVES);
+  if constexpr (BWD) {
+    hipLaunchKernelGGL((scan_bwd_tile_kernel<S, VW>), grid, block, 0, st, p);
   } else {
-    hipLaunchKernelGGL((scan_fwd_kernel<S, VW>), grid, block, lds, st, p);
+    hipLaunchKernelGGL((scan_fwd_tile_kernel<S, VW>), grid, block, 0, st, p);
   }
   return PPO_OK;
 }
@@ -504,38 +590,20 @@ template <bool BWD>
 int dispatch(hipStream_t st, int dtype, ScanArgs p, int batch, const char* what) {
   // 4 features per lane where the rows allow (16-byte float32 or 8-byte bf16
   // accesses; for bf16, 8 per lane would halve the waves in flight).
-  // Time chunks re-read their operands, so they are used only when the lanes
-  // give too few waves: then enough chunks for twice that, at most 16, each
-  // at least 8 steps long.
   const int esize = dtype == SCAN_F32 ? 4 : 2;
   const void* ptrs[8] = {p.a, p.b, p.h, p.init, p.out, p.da, p.dinit, p.reset};
   bool vec = p.F % 4 == 0;
   for (const void* q : ptrs)
     if (q && !aligned(q, 4 * esize)) vec = false;
-  const int VW = vec ? 4 : 1;
-  const int64_t waves = (int64_t)batch * ppo::ceil_div(ppo::ceil_div(p.F, VW), 64);
-  if (p.steps > RL && p.steps <= RL * MAX_CHUNKS) {
-    // register-resident chunks of RL steps: no re-read, every load in flight at once
-    p.chunk = RL;
-    if (dtype == SCAN_F32) {
-      if (vec) launch_reg<float, 4, BWD>(st, p, batch); else launch_reg<float, 1, BWD>(st, p, batch);
-    } else {
-      if (vec) launch_reg<uint16_t, 4, BWD>(st, p, batch); else launch_reg<uint16_t, 1, BWD>(st, p, batch);
-    }
-    return ppo::check_launch(what);
-  }
-  // bf16 rows carry half the bytes per load, so bf16 wants more waves in
-  // flight before the re-read of a second pass stops paying (measured on
-  // [1024, 64, 256]: float32 forward 49 -> 33 us without chunks, bf16 forward
-  // 44 -> 34 us with two)
-  const int64_t enough = dtype == SCAN_F32 ? 512 : 2048;
-  int C = waves >= enough ? 1 : (int)std::min<int64_t>(MAX_CHUNKS, ppo::ceil_div64(2 * enough, waves));
-  C = std::max(1, std::min(C, p.steps / 8));
-  p.chunk = ppo::ceil_div(p.steps, C);
+  // up to 128 steps one register-resident tile (every load of the sequence in
+  // flight at once), longer sequences tile after tile
+  const bool one = p.steps <= RL * MAX_CHUNKS;
   if (dtype == SCAN_F32) {
-    if (vec) launch<float, 4, BWD>(st, p, batch); else launch<float, 1, BWD>(st, p, batch);
+    if (vec) one ? launch_reg<float, 4, BWD>(st, p, batch) : launch_tile<float, 4, BWD>(st, p, batch);
+    else one ? launch_reg<float, 1, BWD>(st, p, batch) : launch_tile<float, 1, BWD>(st, p, batch);
   } else {
-    if (vec) launch<uint16_t, 4, BWD>(st, p, batch); else launch<uint16_t, 1, BWD>(st, p, batch);
+    if (vec) one ? launch_reg<uint16_t, 4, BWD>(st, p, batch) : launch_tile<uint16_t, 4, BWD>(st, p, batch);
+    else one ? launch_reg<uint16_t, 1, BWD>(st, p, batch) : launch_tile<uint16_t, 1, BWD>(st, p, batch);
   }
   return ppo::check_launch(what);
 }
@@ -550,7 +618,7 @@ PPO_EXPORT int ppo_linear_scan_fwd(void* stream, int dtype, const void* a, const
   if (batch == 0 || steps == 0 || features == 0) return PPO_OK;
   if (!a || !b || !init || !out) return ppo::set_error(PPO_ERR_ARG, "ppo_linear_scan_fwd: null buffer");
   if (batch > 65535) return ppo::set_error(PPO_ERR_ARG, "ppo_linear_scan_fwd: batch above 65535");
-  ScanArgs p{a, b, nullptr, init, out, nullptr, nullptr, steps, features, 0, nullptr, nullptr};
+  ScanArgs p{a, b, nullptr, init, out, nullptr, nullptr, steps, features, nullptr, nullptr};
   return dispatch<false>(ppo::as_stream(stream), dtype, p, batch, "ppo_linear_scan_fwd");
 }
 
@@ -562,7 +630,7 @@ PPO_EXPORT int ppo_ssm_scan_fwd(void* stream, int dtype, const void* a, const vo
   if (batch == 0 || steps == 0 || features == 0) return PPO_OK;
   if (!a || !b || !done || !carry || !out) return ppo::set_error(PPO_ERR_ARG, "ppo_ssm_scan_fwd: null buffer");
   if (batch > 65535) return ppo::set_error(PPO_ERR_ARG, "ppo_ssm_scan_fwd: batch above 65535");
-  ScanArgs p{a, b, nullptr, carry, out, nullptr, nullptr, steps, features, 0, done, reset};
+  ScanArgs p{a, b, nullptr, carry, out, nullptr, nullptr, steps, features, done, reset};
   return dispatch<false>(ppo::as_stream(stream), dtype, p, batch, "ppo_ssm_scan_fwd");
 }
 
@@ -576,7 +644,7 @@ PPO_EXPORT int ppo_linear_scan_bwd(void* stream, int dtype, const void* a, const
   if (!a || !h || !init || !cot || !da || !db || !dinit)
     return ppo::set_error(PPO_ERR_ARG, "ppo_linear_scan_bwd: null buffer");
   if (batch > 65535) return ppo::set_error(PPO_ERR_ARG, "ppo_linear_scan_bwd: batch above 65535");
-  ScanArgs p{a, cot, h, init, db, da, dinit, steps, features, 0, nullptr, nullptr};
+  ScanArgs p{a, cot, h, init, db, da, dinit, steps, features, nullptr, nullptr};
   return dispatch<true>(ppo::as_stream(stream), dtype, p, batch, "ppo_linear_scan_bwd");
 }
 
@@ -590,6 +658,6 @@ PPO_EXPORT int ppo_ssm_scan_bwd(void* stream, int dtype, const void* a, const vo
   if (!a || !h || !done || !carry || !cot || !da || !db || !dcarry)
     return ppo::set_error(PPO_ERR_ARG, "ppo_ssm_scan_bwd: null buffer");
   if (batch > 65535) return ppo::set_error(PPO_ERR_ARG, "ppo_ssm_scan_bwd: batch above 65535");
-  ScanArgs p{a, cot, h, carry, db, da, dcarry, steps, features, 0, done, reset};
+  ScanArgs p{a, cot, h, carry, db, da, dcarry, steps, features, done, reset};
   return dispatch<true>(ppo::as_stream(stream), dtype, p, batch, "ppo_ssm_scan_bwd");
 }

@@ -173,3 +173,49 @@ def test_ssm_without_dones_is_the_plain_scan():
     a, b, carry = problem(21, (4, 64, 256))
     done = torch.zeros((4, 64), dtype=torch.bool, device="cuda")
     torch.testing.assert_close(ssm_scan(a, b, done, carry), scan(a, b, carry), rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("batch, steps, features, dtype, offset", [
+    (3, 129, 256, torch.float32, 0), (2, 128 + 64, 100, torch.bfloat16, 0), (1, 1000, 7, torch.float32, 0),
+    (2, 257, 260, torch.float32, 1), (5, 500, 16, torch.bfloat16, 1), (130, 191, 48, torch.bfloat16, 0)])
+@pytest.mark.parametrize("resets", [False, True])
+def test_long_sequences_run_tile_after_tile(batch, steps, features, dtype, offset, resets):
+    """Sequences past one register-resident tile of 128 steps (ragged last
+    tiles, widths and alignments the vector accesses cannot take): forward and
+    gradients against the float64 recurrence, with episode resets at the tile
+    edges among others."""
+    g = torch.Generator(device="cuda").manual_seed(steps + features)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    def leaf(x):
+        flat = torch.empty(x.numel() + offset, dtype=dtype, device="cuda")
+        flat[offset:] = x.to(dtype).reshape(-1)
+        return flat[offset:].view(x.shape).requires_grad_(True)
+    a = leaf(torch.rand(batch, steps, features, device="cuda", generator=g) * 0.9 + 0.05)
+    b, init = leaf(r(batch, steps, features)), leaf(r(batch, features))
+    done = torch.zeros(batch, steps, dtype=torch.bool, device="cuda")
+    reset = r(batch, features).to(dtype)
+    if resets:
+        done |= torch.rand(batch, steps, device="cuda", generator=g) < 0.02
+        done[:, [0, 63, 64, steps - 1]] = True
+    cot = r(batch, steps, features).to(dtype)
+    h = ssm_scan(a, b, done, init, reset) if resets else scan(a, b, init)
+    grads = torch.autograd.grad(h, (a, b, init), cot)
+    A, B, I, R, W = (x.detach().double().cpu() for x in (a, b, init, reset, cot))
+    D = done.cpu()[:, :, None]
+    if resets:
+        B = torch.where(D, B + A * R[:, None], B)
+        A = torch.where(D, 0.0, A)
+    want, s = torch.empty_like(A), I
+    for t in range(steps):
+        s = A[:, t] * s + B[:, t]
+        want[:, t] = s
+    db, d = torch.empty_like(A), torch.zeros_like(I)
+    for t in range(steps - 1, -1, -1):
+        d = W[:, t] + (A[:, t + 1] * d if t + 1 < steps else 0.0)
+        db[:, t] = d
+    prev = torch.cat([I[:, None], want[:, :-1]], 1)
+    da = torch.where(D, R[:, None] * db, db * prev) if resets else db * prev
+    rel = 2e-6 if dtype == torch.float32 else 1e-2   # bf16: 2^-8 per stored value, products of two of them
+    for got, exp in zip((h, *grads), (want, da, db, db[:, 0] * A[:, 0])):
+        got = got.detach().double().cpu()
+        assert float((got - exp).norm()) <= rel * float(exp.norm())
