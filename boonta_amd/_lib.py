@@ -111,6 +111,10 @@ SIGNATURES = {
                                          I, I, P, P, I64, P, I64, P, I, P, I64, P, I64, P, I, I, P, P, P, P, P, P,
                                          P, I, P, I64, P, I64, I, P, I64, P, I64, P, P, P, P, P, P, F, I, F, F, F,
                                          I64]),
+    "ppo_mlp_act_fwd_head_loss_bwd_f32": (I, [P, I, I, P, I64, P, I, I, P, I64, P, P, I64, I, I64, I64, P,
+                                              I, I, P, P, I64, P, I64, P, I, P, I64, P, I64, P, I, I, P, P, P, P, P,
+                                              P, P, I, P, I64, P, I64, I, P, I64, P, I64, P, P, P, P, P, P, F, I, F,
+                                              F, F, I64]),
     "ppo_mlp_ln_fwd_head_loss_bwd_f32": (I, [P, I, I, P, I64, P, I, I, P, I64, I64, P, P, P, P, P, I64, P, P, F, I,
                                              I64, I64, I64, I64, P, I64,
                                              I, I, P, P, I64, P, I64, P, I, P, I64, P, I64, P, I, I, P, P, P, P, P,

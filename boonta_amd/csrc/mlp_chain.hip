@@ -174,36 +174,39 @@ __device__ __forceinline__ void contract(floatx4 (&acc)[4], const float* xrow, b
 // over the same rows (the head input read from LDS instead of HBM), so the
 // results are the same bits; the two towers write disjoint entries of each
 // 16-row block's partials.
-constexpr int HEAD_NB = MC_F / 64;  // 16-feature blocks per wave in the head phases
+constexpr int HEAD_NB = MC_F / 64;  // 16-feature blocks per wave in the head phases (256-wide towers)
 
 // A lane's head parameters for the phases below: the B operands of phase A
 // and C1 (actor) or of phase A and the value weights of C1 (critic), read
 // from the tower's head kernel [256][ld] that the workgroup copied to LDS
 // (hk) at its start.
+template <int NB>
 struct HeadW {
-  float wA[HEAD_NB][4], bT[HEAD_NB][4], wcf[HEAD_NB];
+  float wA[NB][4], bT[NB][4], wcf[NB];
 };
 
-// Copies the tower's head kernel ([256][ld] floats, 256-byte aligned: ld KB)
-// straight into LDS, 1 KB per wave copy; the copies complete in order with
-// the chain's own loads.
+// Copies the tower's head kernel ([64 NB][ld] floats, ld a multiple of 4,
+// 256-byte aligned: ld NB / 4 KB) straight into LDS, 1 KB per wave copy; the
+// copies complete in order with the chain's own loads.
+template <int NB = HEAD_NB>
 __device__ __forceinline__ void copy_head_w(const HeadLossParams& hp, bool actor, float* hk) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const char* src = reinterpret_cast<const char*>(actor ? hp.wa : hp.wc);
   const int ld = actor ? (int)hp.ldwa : (int)hp.ldwc;
-  for (int c = wave; c < ld; c += MC_THREADS / 64)
+  for (int c = wave; c < ld * NB / 4; c += MC_THREADS / 64)
     ppo::lds_copy16(src + 1024 * c + 16 * lane, reinterpret_cast<char*>(hk) + 1024 * c);
 }
 
-__device__ __forceinline__ void load_head_w(const HeadLossParams& hp, bool actor, const float* hk, HeadW& w) {
+template <int NB>
+__device__ __forceinline__ void load_head_w(const HeadLossParams& hp, bool actor, const float* hk, HeadW<NB>& w) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int li = lane & 15;
   const int kq = lane >> 4;
   const int ja = min(li, (int)hp.ldwa - 1);
 #pragma unroll
-  for (int i = 0; i < HEAD_NB; ++i) {
+  for (int i = 0; i < NB; ++i) {
     const int fb = 16 * (wave + 4 * i);
     const int f = fb + li;
     w.wcf[i] = actor ? 0.f : hk[f * hp.ldwc];
@@ -220,12 +223,16 @@ __device__ __forceinline__ void load_head_w(const HeadLossParams& hp, bool actor
   }
 }
 
-template <int PART>
-__device__ __forceinline__ void chain_head(const HeadLossParams& hp, const float (*sX)[SX_PITCH],
-                                           const LaneIn (&lin)[1], const HeadW& w, float (*s_part)[MC_ROWS][LDO],
-                                           float (*s_dout)[LDO], double (*s_st)[NSTAT], float (*s_dsc)[16]) {
+// ACT: the activation whose derivative (at the head input, its output) the
+// input cotangent is multiplied by; with one the result also replaces the
+// head input in the tile sX (every wave holds its share in registers by then).
+template <int PART, int NB = HEAD_NB, int ACT = ACT_NONE>
+__device__ __forceinline__ void chain_head(const HeadLossParams& hp, float (*sX)[64 * NB + 4],
+                                           const LaneIn (&lin)[1], const HeadW<NB>& w, float (*s_part)[MC_ROWS][LDO],
+                                           float (*s_dout)[LDO], double (*s_st)[NSTAT], float (*s_dsc)[16],
+                                           bool to_tile = false) {
   constexpr bool ACTOR = PART == PART_ACTOR;
-  constexpr int NB = HEAD_NB;
+  constexpr int F = 64 * NB;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int li = lane & 15;
@@ -283,12 +290,15 @@ __device__ __forceinline__ void chain_head(const HeadLossParams& hp, const float
       const int f = fb + li;
       const floatx4 g = ppo_hl::mfma4(a_in, w.bT[i], z4);
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (liveq[v]) hp.dha[rowq[v] * hp.lddha + f] = g[v];
+      for (int v = 0; v < 4; ++v) {
+        const float d = ACT == ACT_NONE ? g[v] : g[v] * ppo::act_grad(ACT, h2[i][v]);
+        if (liveq[v]) hp.dha[rowq[v] * hp.lddha + f] = d;
+        if (to_tile) sX[4 * kq + v][f] = liveq[v] ? d : 0.f;
+      }
       const floatx4 gw = ppo_hl::mfma4(floatx4{h2[i][0], h2[i][1], h2[i][2], h2[i][3]}, dq, z4);
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        if (li < (int)hp.ldwa) hp.wpart_a[(blk * MC_F + fb + 4 * kq + v) * hp.ldwa + li] = gw[v];
+        if (li < (int)hp.ldwa) hp.wpart_a[(blk * F + fb + 4 * kq + v) * hp.ldwa + li] = gw[v];
     }
   } else {
     float dvq[4];
@@ -299,15 +309,19 @@ __device__ __forceinline__ void chain_head(const HeadLossParams& hp, const float
       const int fb = 16 * (wave + 4 * i);
       const int f = fb + li;
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (liveq[v]) hp.dhc[rowq[v] * hp.lddhc + f] = dvq[v] * w.wcf[i];
+      for (int v = 0; v < 4; ++v) {
+        const float g = dvq[v] * w.wcf[i];
+        const float d = ACT == ACT_NONE ? g : g * ppo::act_grad(ACT, h2[i][v]);
+        if (liveq[v]) hp.dhc[rowq[v] * hp.lddhc + f] = d;
+        if (to_tile) sX[4 * kq + v][f] = liveq[v] ? d : 0.f;
+      }
       float wv[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) wv[q] = li == 0 ? dvq[q] : 0.f;
       const floatx4 gc = ppo_hl::mfma4(floatx4{h2[i][0], h2[i][1], h2[i][2], h2[i][3]}, wv, z4);
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        if (li < (int)hp.ldwc) hp.wpart_c[(blk * MC_F + fb + 4 * kq + v) * hp.ldwc + li] = li == 0 ? gc[v] : 0.f;
+        if (li < (int)hp.ldwc) hp.wpart_c[(blk * F + fb + 4 * kq + v) * hp.ldwc + li] = li == 0 ? gc[v] : 0.f;
     }
   }
 }
@@ -498,7 +512,7 @@ __device__ __forceinline__ void mlp_ln_fwd_body(const FwdArgs& p, const HeadLoss
     // them explicitly (the compiler does not track them), then meet
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    HeadW hw;
+    HeadW<HEAD_NB> hw;
     load_head_w(hp, t == 0, s_hk, hw);
     if (t == 0) chain_head<PART_ACTOR>(hp, sX, lin, hw, s_part, s_dout, s_st, s_dsc);
     else chain_head<PART_CRITIC>(hp, sX, lin, hw, s_part, s_dout, s_st, s_dsc);
@@ -684,6 +698,259 @@ __global__ void __launch_bounds__(MC_THREADS) mlp_ln_fwd_bwd_kernel(FwdArgs p, H
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   mlp_ln_bwd_body<ACT>(b);
+}
+
+// ---------------------------------------------------------------------------
+// Towers of plain Dense -> activation layers (no LayerNorm), F = 64, 128 or 256
+// features wide: forward, heads + loss and the torso backward of an actor /
+// critic pair in one launch.  A workgroup owns 16 rows of one tower; wave w of
+// NW holds 16 NB = F / NW features, block j's column li being feature 16 NB w +
+// NB li + j.  The layers run back to back on the LDS tile; the activations'
+// derivatives need only the outputs (relu, tanh), which the backward reads back
+// where its own lane wrote them, so there are no statistics and no transposed
+// kernels: dX = dZ W^T reads W along its rows (64-byte pieces), one contraction
+// per inner layer.  What bounds it: every workgroup streams the kernels from L2
+// for 16 rows (about 40 bytes a clock per CU) beside their fp32 MFMAs, 6-7 us a
+// 256 x 256 contraction (8 and 16 waves a workgroup were no faster, 38 and 56 us
+// against 37), and for small towers latency.  2 x 256 tanh towers over 2048 rows
+// of 87 inputs: seven launches of 72 us before, one of 37; 2 x 64 towers over
+// 128 rows of 4: 46 us, 11 (four waves; 128 wide on eight: 17.1 us, on four 18.4).
+struct ActArgs {
+  const float* X;  // layer 0 input rows (row r is X[idx[r]] when idx is non-null)
+  int64_t ldx;
+  const int32_t* idx;
+  int M, K0, L;
+  int64_t ld;      // row pitch of Y and dZ (the kernels' is 64 NB)
+  const float* W[MC_MAXL];
+  const float* bias[MC_MAXL];
+  float* Y[MC_MAXL];
+  float* dZ[MC_MAXL];
+  int64_t tP, tR;  // element strides from tower 0's parameters and rows to tower 1's
+};
+
+template <int NB> struct VecOf;
+template <> struct VecOf<1> { typedef float type; };
+template <> struct VecOf<2> { typedef float type __attribute__((ext_vector_type(2))); };
+template <> struct VecOf<4> { typedef floatx4 type; };
+
+template <int NB>
+__device__ __forceinline__ void load_nb(const float* p, float (&v)[NB]) {
+  const typename VecOf<NB>::type x = *reinterpret_cast<const typename VecOf<NB>::type*>(p);
+  if constexpr (NB == 1) v[0] = x;
+  else
+#pragma unroll
+    for (int j = 0; j < NB; ++j) v[j] = x[j];
+}
+
+template <int NB>
+__device__ __forceinline__ void store_nb(float* p, const float (&v)[NB]) {
+  typename VecOf<NB>::type x;
+  if constexpr (NB == 1) x = v[0];
+  else
+#pragma unroll
+    for (int j = 0; j < NB; ++j) x[j] = v[j];
+  *reinterpret_cast<typename VecOf<NB>::type*>(p) = x;
+}
+
+// acc += A[16 rows][K] W[K][columns c ..]: chunk q of 16 reduction elements as
+// four dependent MFMAs per block, lane group kq taking k = 16 q + 4 kq + s.
+// LDSA: A from the tile row (K = 64 NB), else from global rows.  CH chunks are
+// loaded at a time, the next ones ahead of this set's MFMAs.
+// The kernels' row pitch is F, so a lane's loads take one 32-bit offset from a
+// uniform base each.
+template <int F, int NB, bool LDSA, bool VA, int CH>
+__device__ __forceinline__ void act_contract(floatx4 (&acc)[NB], const float* arow, bool a_live, const float* W, int K,
+                                             int kq, int c) {
+  float a[2][CH][4], w[2][CH][4][NB];
+  auto load = [&](int set, int k0) {
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      const int kb = k0 + 16 * q + 4 * kq;
+      if (LDSA || VA) {
+        // (global rows: a pitch of at least K rounded up to 4)
+        const floatx4 x = *reinterpret_cast<const floatx4*>(arow + (LDSA || (a_live && kb < K) ? kb : 0));
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[set][q][s] = LDSA || (a_live && kb + s < K) ? x[s] : 0.f;
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const bool in = a_live && kb + s < K;
+          const float x = arow[in ? kb + s : 0];
+          a[set][q][s] = in ? x : 0.f;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (LDSA) {
+          load_nb<NB>(W + (k0 + 16 * q + s) * F + (uint32_t)(4 * kq * F + c), w[set][q][s]);
+        } else {
+          const bool in = kb + s < K;
+          load_nb<NB>(W + (uint32_t)(min(kb + s, K - 1) * F + c), w[set][q][s]);
+#pragma unroll
+          for (int j = 0; j < NB; ++j) w[set][q][s][j] = in ? w[set][q][s][j] : 0.f;
+        }
+      }
+    }
+  };
+  auto mma = [&](int set) {
+#pragma unroll
+    for (int q = 0; q < CH; ++q)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][q][s], w[set][q][s][j], acc[j], 0, 0, 0);
+  };
+  load(0, 0);
+#pragma unroll 1
+  for (int k0 = 0; k0 < K; k0 += 32 * CH) {
+    const bool second = k0 + 16 * CH < K;
+    if (second) load(1, k0 + 16 * CH);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!second) break;
+    if (k0 + 32 * CH < K) load(0, k0 + 32 * CH);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// acc += D[16 rows][F] W^T: output feature c + j reads W's row c + j along the
+// reduction.
+template <int F, int NB, int CH>
+__device__ __forceinline__ void act_contract_t(floatx4 (&acc)[NB], const float* lds_row, const float* W, int kq,
+                                               int c) {
+  floatx4 a[2][CH], w[2][CH][NB];
+  auto load = [&](int set, int k0) {
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+      const int kb = k0 + 16 * q + 4 * kq;
+      a[set][q] = *reinterpret_cast<const floatx4*>(lds_row + kb);
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        w[set][q][j] =
+            *reinterpret_cast<const floatx4*>(W + (j * F + k0 + 16 * q) + (uint32_t)(c * F + 4 * kq));
+    }
+  };
+  auto mma = [&](int set) {
+#pragma unroll
+    for (int q = 0; q < CH; ++q)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][q][s], w[set][q][j][s], acc[j], 0, 0, 0);
+  };
+  load(0, 0);
+#pragma unroll
+  for (int k0 = 0; k0 < F; k0 += 32 * CH) {
+    if (k0 + 16 * CH < F) load(1, k0 + 16 * CH);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (k0 + 16 * CH >= F) break;
+    if (k0 + 32 * CH < F) load(0, k0 + 32 * CH);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+template <int F, int NW, int ACT, bool VA>
+__global__ void __launch_bounds__(64 * NW) mlp_act_kernel(ActArgs p, HeadLossParams hp) {
+  constexpr int NB = F / (16 * NW);  // a wave's 16-feature blocks in the layers
+  constexpr int HB = F / 64;         // and of each of the four head waves
+  static_assert(NB * 16 * NW == F && NW >= 4, "four waves run the heads");
+  constexpr int CH = 4;  // a 64-deep set of loads ahead of the MFMAs
+  __shared__ __attribute__((aligned(16))) float sX[MC_ROWS][F + 4];
+  __shared__ __attribute__((aligned(16))) float s_part[4][MC_ROWS][LDO];
+  __shared__ __attribute__((aligned(16))) float s_dout[MC_ROWS][LDO];
+  __shared__ double s_st[MC_ROWS][NSTAT];
+  __shared__ float s_dsc[MC_ROWS][16];
+  __shared__ __attribute__((aligned(1024))) float s_hk[F * 16];  // the tower's head kernel
+  const int64_t t = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int li = lane & 15;
+  const int kq = lane >> 4;
+  const int r0 = blockIdx.x * MC_ROWS;
+  const int c = 16 * NB * wave + NB * li;
+  const int ra = r0 + li;
+  const bool a_live = ra < p.M;
+  const float* xrow = p.X + (a_live ? (int64_t)(p.idx ? p.idx[ra] : ra) * p.ldx : 0);
+  LaneIn lin[1];
+  if (wave < 4) {
+    lane_samples(hp, r0, threadIdx.x, lin);
+    copy_head_w<HB>(hp, t == 0, s_hk);
+  }
+
+  for (int l = 0; l < p.L; ++l) {
+    if (wave < 4 && l == p.L - 1) lane_gathers(hp, threadIdx.x & 15, lin);
+    const float* W = p.W[l] + t * p.tP;
+    float bias[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) bias[j] = 0.f;
+    if (p.bias[l]) load_nb<NB>(p.bias[l] + t * p.tP + c, bias);
+    floatx4 acc[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (l == 0)
+      act_contract<F, NB, false, VA, CH>(acc, xrow, a_live, W, p.K0, kq, c);
+    else
+      act_contract<F, NB, true, true, CH>(acc, &sX[li][0], true, W, F, kq, c);
+    __syncthreads();  // every wave is past its reads of the tile
+    float* Y = p.Y[l] + t * p.tR;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int rr = 4 * kq + v;
+      float y[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) y[j] = ppo::act_fwd(ACT, acc[j][v] + bias[j]);
+      store_nb<NB>(&sX[rr][c], y);
+      if (r0 + rr < p.M) store_nb<NB>(Y + (int64_t)(r0 + rr) * p.ld + c, y);
+    }
+    __syncthreads();
+  }
+
+  // heads and loss; the last layer's dZ goes to memory and into the tile (the
+  // head kernel's copies, issued first, are long complete)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (wave < 4) {
+    HeadW<HB> hw;
+    load_head_w<HB>(hp, t == 0, s_hk, hw);
+    if (t == 0) chain_head<PART_ACTOR, HB, ACT>(hp, sX, lin, hw, s_part, s_dout, s_st, s_dsc, true);
+    else chain_head<PART_CRITIC, HB, ACT>(hp, sX, lin, hw, s_part, s_dout, s_st, s_dsc, true);
+  } else {
+    __syncthreads();  // chain_head's two barriers
+    __syncthreads();
+  }
+
+  for (int l = p.L - 1; l > 0; --l) {
+    __syncthreads();  // dZ of layer l is in the tile
+    floatx4 acc[NB];
+    float y[4][NB];  // this lane's outputs of layer l - 1
+    const float* Y = p.Y[l - 1] + t * p.tR;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) load_nb<NB>(Y + (int64_t)min(r0 + 4 * kq + v, p.M - 1) * p.ld + c, y[v]);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    act_contract_t<F, NB, CH>(acc, &sX[li][0], p.W[l] + t * p.tP, kq, c);
+    __syncthreads();
+    float* dZ = p.dZ[l - 1] + t * p.tR;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int rr = 4 * kq + v;
+      const bool live = r0 + rr < p.M;
+      float d[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) d[j] = live ? acc[j][v] * ppo::act_grad(ACT, y[v][j]) : 0.f;
+      if (l > 1) store_nb<NB>(&sX[rr][c], d);
+      if (live) store_nb<NB>(dZ + (int64_t)(r0 + rr) * p.ld + c, d);
+    }
+  }
 }
 
 bool aligned16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
@@ -921,5 +1188,74 @@ PPO_EXPORT int ppo_mlp_ln_fwd_head_loss_bwd_f32(
     default: PPO_CHAIN_FB(ACT_NONE) break;
   }
 #undef PPO_CHAIN_FB
+  return ppo::check_launch(name);
+}
+
+// Forward of an actor / critic pair of L plain Dense(F) -> activation layers
+// (F = 64, 128 or 256; relu, tanh or none; towers as two blocks of one
+// layout, stride_params and stride_rows elements apart), their fused heads +
+// PPO loss and the torso backward, in one launch: Y[l], the head partials and
+// statistics of ppo_head_loss_f32, and dZ[l] of every layer (dha = dZ[L - 1],
+// dhc = dha + stride_rows: the head inputs' cotangents times the activation's
+// derivative at ha = Y[L - 1]).  The head arguments are ppo_head_loss_f32's,
+// for separate heads over the last layer's outputs and a minibatch whose
+// partials are kept per 16-row block.
+PPO_EXPORT int ppo_mlp_act_fwd_head_loss_bwd_f32(
+    void* stream, int towers, int L, const float* X, int64_t ldx, const int32_t* rows_idx, int M, int K0,
+    const float* const* W, int64_t ldw0, const float* const* bias, float* const* Y, int64_t ld, int act,
+    int64_t stride_params, int64_t stride_rows, float* const* dZ, int dist, int rows, const int32_t* idx,
+    const float* ha, int64_t ldha, const float* wa, int64_t ldwa, const float* ba, int na, const float* hc, int64_t ldhc,
+    const float* wc, int64_t ldwc, const float* bc, int F, int A, const float* scale_param, const int32_t* action_i,
+    const float* action_f, const float* old_logp, const float* old_value, const float* adv, const float* ret, int act_a,
+    const float* aux_a, int64_t ldaux_a, float* dha, int64_t lddha, int act_c, const float* aux_c, int64_t ldaux_c,
+    float* dhc, int64_t lddhc, float* wpart_a, float* bpart_a, float* wpart_c, float* bpart_c, float* dscale_partial,
+    double* stats_partial, float clip_eps, int clip_value_loss, float ent_coef, float vf_coef, float temperature,
+    int64_t sample_stride) {
+  const char* name = "ppo_mlp_act_fwd_head_loss_bwd_f32";
+  if (towers != 2 || L < 1 || L > MC_MAXL || M < 0 || K0 < 1 || ldx < K0 || (F != 64 && F != 128 && F != 256) ||
+      ldw0 != F || ld != F || (int64_t)K0 * F > INT32_MAX || (act != ACT_NONE && act != ACT_RELU && act != ACT_TANH) || !X || !W || !bias ||
+      !Y || !dZ || stride_params % 4 || stride_rows % 4)
+    return ppo::set_error(PPO_ERR_ARG, "%s: bad argument (towers=%d L=%d M=%d K0=%d F=%d act=%d)", name, towers, L, M, K0,
+                          F, act);
+  ActArgs a{};
+  a.X = X; a.ldx = ldx; a.idx = rows_idx; a.M = M; a.K0 = K0; a.L = L; a.ld = ld;
+  a.tP = stride_params; a.tR = stride_rows;
+  for (int l = 0; l < L; ++l) {
+    if (!W[l] || !Y[l] || !dZ[l] || !aligned16(W[l]) || (bias[l] && !aligned16(bias[l])) || !aligned16(Y[l]) ||
+        !aligned16(dZ[l]))
+      return ppo::set_error(PPO_ERR_ARG, "%s: layer %d needs 16-byte aligned buffers", name, l);
+    a.W[l] = W[l]; a.bias[l] = bias[l]; a.Y[l] = Y[l]; a.dZ[l] = dZ[l];
+  }
+  HeadLossParams hp;
+  const int rc = head_loss_setup(hp, name, dist, rows, idx, ha, ldha, wa, ldwa, ba, na, hc, ldhc, wc, ldwc, bc, F, A,
+                                 scale_param, action_i, action_f, old_logp, old_value, adv, ret, act_a, aux_a, ldaux_a,
+                                 dha, lddha, act_c, aux_c, ldaux_c, dhc, lddhc, wpart_a, bpart_a, wpart_c, bpart_c,
+                                 dscale_partial, stats_partial, clip_eps, clip_value_loss, ent_coef, vf_coef,
+                                 temperature, nullptr, 1, 1, sample_stride);
+  if (rc != PPO_OK) return rc;
+  if (!hc || act_a != act || act_c != act || rows != M || ha != Y[L - 1] || hc != Y[L - 1] + stride_rows || ldha != ld ||
+      ldhc != ld || dha != dZ[L - 1] || dhc != dha + stride_rows || lddha != ld || lddhc != ld || ldwa % 4 || ldwc % 4 ||
+      ldwa > 16 || ldwc > 16 || (reinterpret_cast<uintptr_t>(wa) & 255) || (reinterpret_cast<uintptr_t>(wc) & 255) ||
+      (M > 0 && ppo_head_loss_blocks(M) != ppo::ceil_div(M, MC_ROWS)))
+    return ppo::set_error(PPO_ERR_ARG, "%s: the heads must read the last layer of both towers (F=%d rows=%d M=%d)", name,
+                          F, rows, M);
+  if (M == 0) return PPO_OK;
+  const bool va = aligned16(X) && ldx % 4 == 0;  // ldx >= K0, so >= K0 rounded up to 4
+  const dim3 grid(ppo::ceil_div(M, MC_ROWS), towers);
+  hipStream_t st = ppo::as_stream(stream);
+#define PPO_ACT_CHAIN(FV, NWV, ACTV)                                                                            \
+  if (va) hipLaunchKernelGGL((mlp_act_kernel<FV, NWV, ACTV, true>), grid, dim3(64 * NWV), 0, st, a, hp);       \
+  else hipLaunchKernelGGL((mlp_act_kernel<FV, NWV, ACTV, false>), grid, dim3(64 * NWV), 0, st, a, hp);
+#define PPO_ACT_CHAIN_W(ACTV)                         \
+  if (F == 64) { PPO_ACT_CHAIN(64, 4, ACTV) }         \
+  else if (F == 128) { PPO_ACT_CHAIN(128, 8, ACTV) }  \
+  else { PPO_ACT_CHAIN(256, 4, ACTV) }
+  switch (act) {
+    case ACT_RELU: PPO_ACT_CHAIN_W(ACT_RELU) break;
+    case ACT_TANH: PPO_ACT_CHAIN_W(ACT_TANH) break;
+    default: PPO_ACT_CHAIN_W(ACT_NONE) break;
+  }
+#undef PPO_ACT_CHAIN_W
+#undef PPO_ACT_CHAIN
   return ppo::check_launch(name);
 }

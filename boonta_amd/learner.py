@@ -219,6 +219,10 @@ def _splits(rows: int, m: int, n: int) -> int:
     return max(1, min(max(1, rows // 128), math.ceil(target / tiles)))
 
 
+# split counts whose sums a grouped weight-gradient launch finishes itself
+FINAL_SPLITS = (1, 2, 3, 4, 6, 8, 12, 16, 32, 64)
+
+
 @dataclass
 class LayerBufs:
     spec: LayerSpec
@@ -352,12 +356,15 @@ def paired_tower_bufs(specs_a, specs_c, rows: int, device, ln_blocks: int | None
     for i, s in enumerate(specs_a):
         # batched over depth and towers in one launch that also finishes the
         # split-K sums (the last split of each tile reads the others'
-        # partials back), fewer splits: half for the first layer, 3/8 for the
-        # later ones (2048-row Gaussian minibatches: 8 and 6 splits, 5.08 M
-        # samples/s, against 5.05 M with 16 and 8)
+        # partials back), fewer splits: 3/4 for the first layer, half for the
+        # later ones (2048-row minibatches, 12 and 8 splits: 2-layer tanh towers
+        # 2227 us per update of 32, 8 / 6 splits 2293, 16 / 12 2248; 4-layer
+        # LayerNorm towers 3199, 3210, 3268)
         sp = _splits(rows, s.dense.fin, s.ld)
         if grouped_dw:
-            sp = sp // 2 if i == 0 else 3 * sp // 8
+            # (a count the launch's finishing sums are compiled for)
+            sp = 3 * sp // 4 if i == 0 else sp // 2
+            sp = max(f for f in FINAL_SPLITS if f <= max(1, sp))
         A[i].splits = C[i].splits = max(1, sp)
         if ln[i]:
             A[i].lnblocks = C[i].lnblocks = blocks
@@ -700,16 +707,20 @@ class MLPExecutor(ForwardChain):
         # towers of 256-wide LayerNorm layers (one activation, one epsilon)
         # run each direction of the whole torso chain in one launch
         self.chain_ln = bool(self.pair) and self.CHAIN and self._chainable(program.actor_layers)
+        # towers of plain Dense -> activation layers run their forward, heads +
+        # loss and torso backward in one launch
+        self.chain_act = bool(self.pair) and self.CHAIN and self._act_chainable(program, mb)
+        self.chain_dw = self.chain_ln or self.chain_act  # their weight gradients in one launch
         # observation rows whose width is not a multiple of four: a zero-padded
         # copy per update lets the first layer's weight gradient run on the
         # copy-fed GEMM over the padded width (the Gaussian workload's 87
         # features: 10.2 us per step on the register-staged kernel)
         fin0 = program.actor_layers[0].dense.fin if program.actor_layers else 0
-        self.obs_pad = (fin0 + 3) // 4 * 4 if self.chain_ln and fin0 % 4 != 0 and fin0 == self.obs_dim else 0
+        self.obs_pad = (fin0 + 3) // 4 * 4 if self.chain_dw and fin0 % 4 != 0 and fin0 == self.obs_dim else 0
         if self.pair:
             lnb = _lib.load().ppo_mlp_ln_bwd_blocks(mb) if self.chain_ln else None
             self.actor, self.critic = paired_tower_bufs(program.actor_layers, program.critic_layers, mb, dev, lnb,
-                                                        grouped_dw=self.chain_ln, fin0_pad=self.obs_pad)
+                                                        grouped_dw=self.chain_dw, fin0_pad=self.obs_pad)
         else:
             self.actor = [layer_bufs(s, mb, True) for s in program.actor_layers]
             self.critic = [layer_bufs(s, mb, True) for s in program.critic_layers]
@@ -762,6 +773,8 @@ class MLPExecutor(ForwardChain):
             L = len(self.actor)
             self.WT = torch.zeros(max(L - 1, 1), 2, 256, 256, **f32)
             self._chain_tables()
+        if self.chain_act:
+            self._act_tables()
         ha, hc = program.head_a, program.head_c
         lib = _lib.load()
         self.fused = self._can_fuse(program)
@@ -876,6 +889,49 @@ class MLPExecutor(ForwardChain):
         return all(s.ln is not None and s.fout == 256 and s.ld == 256 and s.act == s0.act
                    and s.ln["eps"] == s0.ln["eps"] and s.dense.w.ld == 256 for s in layers)
 
+    # plain towers in one launch per step: None where the parameters are on the
+    # device (whose allocations keep the head kernels' 256-byte alignment); True
+    # to record such launches over host memory
+    CHAIN_ACT = None
+
+    def _act_chainable(self, program: Program, mb: int) -> bool:
+        """Towers ppo_mlp_act_fwd_head_loss_bwd_f32 takes: up to
+        ppo_mlp_chain_max_layers() Dense(F) layers (F = 64, 128 or 256) of one
+        activation (relu, tanh or none) and no LayerNorm under the fused heads,
+        and a minibatch whose head partials are kept per 16-row block."""
+        layers, lib = program.actor_layers, _lib.load()
+        if not (self.flat.P.is_cuda if self.CHAIN_ACT is None else self.CHAIN_ACT):
+            return False
+        if len(layers) > lib.ppo_mlp_chain_max_layers() or self._ratio_out() is not None:
+            return False
+        s0 = layers[0]
+        F = s0.fout
+        if F not in (64, 128, 256) or s0.act not in ("relu", "tanh", None):
+            return False
+        if any(s.ln is not None or s.fout != F or s.ld != F or s.dense.w.ld != F or s.act != s0.act
+               or (i > 0 and s.dense.fin != F) for i, s in enumerate(layers)):
+            return False
+        # the launch copies each head kernel into LDS from its 256-byte aligned start
+        base = self.flat.P.data_ptr() if self.flat.P.is_cuda else 0
+        heads = (program.head_a, program.head_c)
+        return (all((base + 4 * h.w.offset) % 256 == 0 and h.fin == F and h.w.ld <= 16 for h in heads)
+                and lib.ppo_head_loss_blocks(mb) == -(-mb // 16))
+
+    def _act_tables(self):
+        """Per-layer pointer tables of the plain towers' launch (kept alive on
+        the executor), and the rows' element stride between the towers."""
+        A, C = self.actor, self.critic
+        view = self.flat.view
+        arr = lambda xs: (ctypes.c_void_p * len(xs))(*xs)
+        keep = {"W": arr([view(lb.spec.dense.w) for lb in A]),
+                "b": arr([view(lb.spec.dense.b) if lb.spec.dense.b is not None else None for lb in A]),
+                "Y": arr([_p(lb.Y) for lb in A]), "dZ": arr([_p(lb.dZ) for lb in A])}
+        rows = _tstride(A[0].Y, C[0].Y)
+        assert all(_tstride(a.Y, c.Y) == rows == _tstride(a.dZ, c.dZ) for a, c in zip(A, C))
+        self._act = {k: ctypes.addressof(v) for k, v in keep.items()}
+        self._act.update(keep=keep, rows=rows)
+        self._dw_groups = self._plan_dw_groups()
+
     def _chain_tables(self):
         """Per-layer pointer tables of the chain launches (ctypes arrays kept
         alive on the executor; the pointers are fixed for its lifetime)."""
@@ -925,10 +981,8 @@ class MLPExecutor(ForwardChain):
     PAIR_DW_GROUP = True
 
     # the paired towers' weight gradients finish their split-K sums in their
-    # grouped launch (no gradient-reduce launch for them); the split counts
-    # that launch supports
+    # grouped launch (no gradient-reduce launch for them)
     DW_FINAL = True
-    FINAL_SPLITS = (1, 2, 3, 4, 6, 8, 12, 16, 32, 64)
 
     def _first_dw_final(self, st, layers, x, ldx, ridx) -> bool:
         """The shared trunk's first-layer weight gradient as a one-problem
@@ -964,7 +1018,7 @@ class MLPExecutor(ForwardChain):
         weight-gradient launch, in its order (layer-major, actor then
         critic), or None when the towers do not take that launch."""
         A, C = self.actor, self.critic
-        if not self.PAIR_DW_GROUP or not self.chain_ln or 2 * len(A) > 8:
+        if not self.PAIR_DW_GROUP or not self.chain_dw or 2 * len(A) > 8:
             return None
         fin0 = self.obs_pad if self.obs_pad else A[0].spec.dense.fin
         return [(fin0 if i == 0 else lb.spec.dense.fin, lb.spec.ld, lb.splits)
@@ -1097,7 +1151,7 @@ class MLPExecutor(ForwardChain):
         for k, lb in enumerate(self.trunk + self.actor + self.critic):
             n0 = len(segs)
             dense_segs(lb.spec.dense, lb.wpart, lb.bpart, lb.splits)
-            if self.chain_ln and k >= len(self.trunk):
+            if self.chain_dw and k >= len(self.trunk):
                 paired.update(range(n0, len(segs)))
             elif k == 0 and self.trunk:
                 first.update(range(n0, len(segs)))
@@ -1151,7 +1205,7 @@ class MLPExecutor(ForwardChain):
         # slots, then the other segments' chunks, reduced in the same launch
         self.dw_final = None
         shapes = self._pair_dw_shapes() if self.DW_FINAL and paired else None
-        if shapes and all(sp in self.FINAL_SPLITS and (i >= 2 or -(-self.mb // sp) <= 512)
+        if shapes and all(sp in FINAL_SPLITS and (i >= 2 or -(-self.mb // sp) <= 512)
                           for i, (_, _, sp) in enumerate(shapes)):
             L = len(shapes)
             T = lib.ppo_gemm_f32_dw_final_slots(L, (ctypes.c_int * L)(*[m for m, _, _ in shapes]),
@@ -1169,7 +1223,7 @@ class MLPExecutor(ForwardChain):
         # (at the largest split count the launch sums that does not exceed the
         # layer's own: the GRU workload's 128 splits of 128 rows become 64)
         lb0 = self.trunk[0] if self.trunk else None
-        sp0 = max([sp for sp in self.FINAL_SPLITS if lb0 is not None and sp <= lb0.splits] or [0])
+        sp0 = max([sp for sp in FINAL_SPLITS if lb0 is not None and sp <= lb0.splits] or [0])
         if (self.DW_FINAL and self.dw_final is None and sp0 > 0 and not self.bf16 and self.fused
                 and self.prog.shared_head and lb0.spec.ln is None and -(-self.mb // sp0) <= 512
                 and lb0.spec.dense.fin % 4 == 0 and lb0.spec.ld % 4 == 0):
@@ -1377,9 +1431,9 @@ class MLPExecutor(ForwardChain):
         (chain_done: the torso chains' backward already ran, in the forward's
         launch; only the weight gradients remain)."""
         D, A, C = self.pair, self.actor, self.critic
-        if self.chain_ln:
-            c = self._chain
+        if self.chain_dw:
             if not chain_done:
+                c = self._chain
                 self._call("ppo_mlp_ln_bwd_f32", st, 2, len(A), _p(A[-1].dY), A[-1].spec.ld, self.mb, c["Z"],
                            c["mean"], c["rstd"], c["g"], c["be"], c["WT"], 256, c["dZ"], A[0].spec.ld, c["part"],
                            self._chain_act, self._chain_rs, self._chain_ss, D, 256 * 256, self._chain_ps)
@@ -1733,6 +1787,14 @@ class MLPExecutor(ForwardChain):
                 self._fwd_layers(st, self.trunk, obs, ldo, idx, mb)
                 self._fused_head_loss(st, idx, step, dist, A, scale_ptr, act_i, act_f)
                 self._bwd_layers(st, self.trunk, obs, ldo, idx, side_dw=True)
+            elif self.chain_act:
+                t, s0, pre = self._act, self.actor[0].spec, self._head_loss_args
+                # (the zero-padded copy's rows take 16-byte loads)
+                x, ldx = (_p(self.OBSP), self.obs_pad) if self.obs_pad else (obs, ldo)
+                self._call("ppo_mlp_act_fwd_head_loss_bwd_f32", st, 2, len(self.actor), x, ldx, idx, mb, s0.dense.fin,
+                           t["W"], s0.dense.w.ld, t["b"], t["Y"], s0.ld, _act(s0.act), self.pair, t["rows"], t["dZ"],
+                           *pre(idx, step, dist, A, scale_ptr, act_i, act_f), self._sample_stride())
+                self._bwd_pair(st, obs, ldo, idx, chain_done=True)
             elif self.pair:
                 if self._chain_head and self._fwd_bwd_fused() and step > 0:
                     # forward, heads + loss and the torso backward in one launch: the

@@ -635,6 +635,26 @@ int ppo_mlp_ln_fwd_head_loss_bwd_f32(
     float* dscale_partial, double* stats_partial, float clip_eps, int clip_value_loss, float ent_coef,
     float vf_coef, float temperature, int64_t sample_stride, float* const* dZ, float* const* partial,
     int64_t stride_part);
+/* An actor / critic pair (towers = 2) of L plain Dense(F) -> activation layers
+ * (F = 64, 128 or 256; relu, tanh or none; no LayerNorm), their fused heads +
+ * PPO loss and the torso backward in one launch: writes Y[l], what
+ * ppo_head_loss_f32 writes for separate heads over the last outputs (ha =
+ * Y[L - 1], hc = ha + stride_rows; act_a = act_c = act; dha = dZ[L - 1], dhc =
+ * dha + stride_rows) and dZ[l] of every layer, all of row pitch ld = F.  The
+ * parameters of tower 1 sit stride_params elements after tower 0's.
+ * Replaces the same reference code as ppo_mlp_ln_fwd_head_loss_bwd_f32 for
+ * torsos without LayerNorm (boonta/algorithms/ppo.py:77-157). */
+int ppo_mlp_act_fwd_head_loss_bwd_f32(
+    void* stream, int towers, int L, const float* X, int64_t ldx, const int32_t* rows_idx, int M, int K0,
+    const float* const* W, int64_t ldw0, const float* const* bias, float* const* Y, int64_t ld, int act,
+    int64_t stride_params, int64_t stride_rows, float* const* dZ, int dist, int rows, const int32_t* idx,
+    const float* ha, int64_t ldha, const float* wa, int64_t ldwa, const float* ba, int na, const float* hc, int64_t ldhc,
+    const float* wc, int64_t ldwc, const float* bc, int F, int A, const float* scale_param, const int32_t* action_i,
+    const float* action_f, const float* old_logp, const float* old_value, const float* adv, const float* ret, int act_a,
+    const float* aux_a, int64_t ldaux_a, float* dha, int64_t lddha, int act_c, const float* aux_c, int64_t ldaux_c,
+    float* dhc, int64_t lddhc, float* wpart_a, float* bpart_a, float* wpart_c, float* bpart_c, float* dscale_partial,
+    double* stats_partial, float clip_eps, int clip_value_loss, float ent_coef, float vf_coef, float temperature,
+    int64_t sample_stride);
 /* ppo_head_loss_f32 that also keeps each row's ratio exp(logp - old_logp),
  * env-major: ratio_out[(s % envs) * steps + s / envs] for the row's sample
  * s = idx[row] = t * envs + env (the new ratio RecurrentPuPO scatters back
