@@ -49,6 +49,9 @@ SIGNATURES = {
     "ppo_step_mlp_max_layers": (I, []),
     "ppo_step_mlp_max_obs": (I, []),
     "ppo_step_mlp_categorical_f32": (I, [P, P, I64, I, I, I, P, P, P, I, P, I64, P, I, P, F, P, P, P]),
+    "ppo_step_towers_max_layers": (I, []),
+    "ppo_step_towers_max_outputs": (I, []),
+    "ppo_step_towers_f32": (I, [P, P, I64, I, I, I, I, P, P, P, P, F, I, P, P, P, I, P, P, F, P, P, P]),
     "ppo_priority_choice_max_envs": (I, []),
     "ppo_priority_choice_f32": (I, [P, P, I64, I, I, F, F, P, I, P, P, P]),
     "ppo_gemm_ln_act_fwd_f32": (I, [P, P, I64, P, P, I64, P, P, P, P, I64, P, I64, P, P, I, I, I, F, I]),

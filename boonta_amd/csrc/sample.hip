@@ -30,6 +30,7 @@
 #include "common.h"
 #include "threefry.h"
 #include "categorical.h"
+#include "gaussian.h"
 
 #include <math.h>
 
@@ -39,47 +40,6 @@ constexpr int GROUP = 16;
 constexpr int THREADS = 256;
 constexpr int ROWS_PER_BLOCK = THREADS / GROUP;
 constexpr int MAX_K = 8;  // columns per lane: A, D <= 128
-constexpr float HALF_LOG_2PI = 0.91893853320467274f;
-
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int o = GROUP / 2; o; o >>= 1) v += __shfl_xor(v, o, GROUP);
-  return v;
-}
-
-__device__ __forceinline__ float softplus_acc(float x) {
-  // jax.nn.softplus = logaddexp(x, 0)
-  return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
-}
-
-__device__ __forceinline__ float erfinv_giles(float x) {
-  float w = -log1pf(-(x * x));
-  float p;
-  if (w < 5.0f) {
-    w = w - 2.5f;
-    p = 2.81022636e-08f;
-    p = 3.43273939e-07f + p * w;
-    p = -3.5233877e-06f + p * w;
-    p = -4.39150654e-06f + p * w;
-    p = 0.00021858087f + p * w;
-    p = -0.00125372503f + p * w;
-    p = -0.00417768164f + p * w;
-    p = 0.246640727f + p * w;
-    p = 1.50140941f + p * w;
-  } else {
-    w = sqrtf(w) - 3.0f;
-    p = -0.000200214257f;
-    p = 0.000100950558f + p * w;
-    p = 0.00134934322f + p * w;
-    p = -0.00367342844f + p * w;
-    p = 0.00573950773f + p * w;
-    p = -0.0076224613f + p * w;
-    p = 0.00943887047f + p * w;
-    p = 1.00167406f + p * w;
-    p = 2.83297682f + p * w;
-  }
-  return fabsf(x) == 1.0f ? x * INFINITY : p * x;
-}
 
 struct CatArgs {
   const float* pref;
@@ -131,26 +91,19 @@ __global__ void __launch_bounds__(THREADS) sample_gaussian_kernel(GaussArgs a) {
   const int j0 = threadIdx.x % GROUP;
   const bool row_ok = r < a.rows;
   const uint32_t k0 = a.key[0], k1 = a.key[1];
-  const float lo = -0.99999994f;  // nextafter(-1, 0)
-  const float span = 1.0f - lo;   // maxval - minval, rounded to float32
   const uint64_t base = (uint64_t)(row_ok ? r : 0) * (uint64_t)a.D;
   float lpx = 0.f, logdet = 0.f;
 #pragma unroll
   for (int k = 0; k < MAX_K; ++k) {
     const int j = j0 + GROUP * k;
     if (row_ok && j < a.D) {
-      const float f = ppo::unit_float(ppo::random_word(k0, k1, base + (uint64_t)j));
-      const float u = fmaxf(lo, f * span + lo);
-      const float eps = 1.41421356237309515f * erfinv_giles(u);
       const float raw = a.lds ? a.scale[(int64_t)r * a.lds + j] : a.scale[j];
-      const float sig = a.temperature * (softplus_acc(raw) + 1e-3f);
-      a.action[(int64_t)r * a.lda + j] = sig * eps + a.mean[(int64_t)r * a.ldm + j];
-      lpx += -0.5f * (eps * eps) - HALF_LOG_2PI;
-      logdet += logf(sig);
+      a.action[(int64_t)r * a.lda + j] =
+          ppo::gauss::draw(a.mean[(int64_t)r * a.ldm + j], raw, k0, k1, base + (uint64_t)j, a.temperature, lpx, logdet);
     }
   }
-  lpx = group_sum(lpx);
-  logdet = group_sum(logdet);
+  lpx = ppo::cat::group_sum(lpx);
+  logdet = ppo::cat::group_sum(logdet);
   if (row_ok && j0 == 0) {
     a.log_prob[r] = lpx - logdet;
     if (a.value) a.value[r] = a.vsrc[(int64_t)r * a.ldv];

@@ -36,8 +36,11 @@ class StepExecutor(ForwardChain):
 
     A float32 shared-trunk MLP of 256-wide Dense layers with one activation
     and a categorical head of at most 15 logits (the discrete Anakin network)
-    steps in one launch, ``ppo_step_mlp_categorical_f32``; ``fused=False``
-    issues the layer-by-layer GEMMs and the sampling launch instead."""
+    steps in one launch, ``ppo_step_mlp_categorical_f32``, and float32 actor
+    and critic towers of one shape (Dense layers of 64, 128 or 256 features, or
+    256 with LayerNorm; at most 16 actor outputs) in ``ppo_step_towers_f32``;
+    ``fused=False`` issues the layer-by-layer GEMMs and the sampling launch
+    instead."""
 
     def __init__(self, program: Program, flat: FlatState, rows: int, fused: bool = True):
         if program.gru is not None:
@@ -63,6 +66,7 @@ class StepExecutor(ForwardChain):
             self.HC = torch.zeros(rows, hc.w.ld, **f32)
         self.KEY = torch.zeros(2, dtype=torch.int32, device=dev)
         self.fused = fused and self._fusable(lib)
+        self.towers = self._tower_tables() if fused and self._towers_fusable(lib) else None
 
     def _fusable(self, lib) -> bool:
         """Whether the one-launch step kernel covers this program."""
@@ -77,6 +81,58 @@ class StepExecutor(ForwardChain):
             return False
         h = prog.head_a
         return h.fin == 256 and h.w.ld <= 16 and prog.head_out == prog.dist["num"] and prog.head_out + 1 <= h.w.ld
+
+    def _towers_fusable(self, lib) -> bool:
+        """Whether the paired towers' one-launch step covers this program: for
+        every number of rows it replaces two launches per layer and three after
+        (4 x 256 LayerNorm + SiLU, 4096 rows: 125 -> 64 us)."""
+        prog = self.prog
+        A, C = prog.actor_layers, prog.critic_layers
+        if (self.bf16 or prog.shared_head or not A or len(A) != len(C) or len(A) > lib.ppo_step_towers_max_layers()
+                or A[0].dense.fin * A[0].fout > 2 ** 31 - 1):
+            return False
+        s0 = A[0]
+        F, ln = s0.fout, s0.ln is not None
+        if F not in ((256,) if ln else (64, 128, 256)) or s0.act not in ("relu", "tanh", None) + (("silu",) if ln else ()):
+            return False
+        for layers in (A, C):
+            for i, s in enumerate(layers):
+                if (s.fout != F or s.ld != F or s.dense.w.ld != F or s.act != s0.act or (s.ln is not None) != ln
+                        or s.dense.fin != (A[0].dense.fin if i == 0 else F) or (ln and s.ln["eps"] != s0.ln["eps"])):
+                    return False
+        ha, hc = prog.head_a, prog.head_c
+        gaussian = prog.dist["kind"] != "categorical"
+        if gaussian and (prog.scale_region is None or prog.dist["dim"] != prog.head_out):
+            return False
+        if not gaussian and prog.dist["num"] != prog.head_out:
+            return False
+        # (the launch loads parameters as 16-byte vectors)
+        base = self.flat.P.data_ptr()
+        regions = [r for layers in (A, C) for s in layers
+                   for r in (s.dense.w, s.dense.b, *((s.ln["scale"], s.ln["bias"]) if ln else ())) if r is not None]
+        return (ha.fin == F and hc.fin == F and hc.fout == 1 and prog.head_out <= lib.ppo_step_towers_max_outputs()
+                and all((base + 4 * r.offset) % 16 == 0 for r in regions))
+
+    def _tower_tables(self) -> dict:
+        """Host arrays of ppo_step_towers_f32's parameter pointers (kept: the
+        flat buffers live as long as this executor)."""
+        prog, view = self.prog, self.flat.view
+        layers = prog.actor_layers + prog.critic_layers
+        heads = (prog.head_a, prog.head_c)
+        vp = lambda xs: (ctypes.c_void_p * len(xs))(*xs)
+        ln = layers[0].ln
+        keep = {"W": vp([view(s.dense.w) for s in layers]),
+                "b": vp([view(s.dense.b) if s.dense.b is not None else None for s in layers]),
+                "g": vp([view(s.ln["scale"]) for s in layers]) if ln else None,
+                "be": vp([view(s.ln["bias"]) for s in layers]) if ln else None,
+                "hw": vp([view(h.w) for h in heads]), "ldh": (ctypes.c_int64 * 2)(*[h.w.ld for h in heads]),
+                "hb": vp([view(h.b) if h.b is not None else None for h in heads])}
+        s0 = layers[0]
+        t = {k: None if v is None else ctypes.addressof(v) for k, v in keep.items()}
+        t.update(keep=keep, args=(len(prog.actor_layers), s0.fout, t["W"], t["b"], t["g"], t["be"],
+                                  float(ln["eps"]) if ln else 0.0, _act(s0.act), t["hw"], t["ldh"], t["hb"],
+                                  prog.head_out, view(prog.scale_region) if prog.scale_region is not None else None))
+        return t
 
     def _head(self, st, x, ldx, h: DenseSpec, out: torch.Tensor):
         """Head Dense on the last features (bias added, no activation)."""
@@ -103,6 +159,10 @@ class StepExecutor(ForwardChain):
             self._call("ppo_step_mlp_categorical_f32", st, obs, ldo, rows, prog.trunk[0].dense.fin, n, ws, lds, bs, _act(prog.trunk[0].act), self.flat.view(h.w), h.w.ld,
                        self.flat.view(h.b) if h.b is not None else None, prog.dist["num"], key, float(temperature),
                        action, log_prob, value)
+            return
+        if self.towers is not None:
+            self._call("ppo_step_towers_f32", st, obs, ldo, rows, prog.actor_layers[0].dense.fin, *self.towers["args"],
+                       key, float(temperature), action, log_prob, value)
             return
         if prog.shared_head:
             x, ldx, _ = self._fwd_layers(st, self.trunk, obs, ldo, None, rows)

@@ -156,6 +156,25 @@ int ppo_step_mlp_categorical_f32(void* stream, const float* obs, int64_t ldo, in
                                  const float* head_w, int64_t ldwh, const float* head_b, int A, const uint32_t* key,
                                  float temperature, int32_t* action, float* log_prob, float* value);
 
+/* The whole PPO.step of an MLP actor-critic with separate torsos of one shape
+ * in one launch (ActorCritic with Sequential actor and critic, network.py:18-49):
+ * `layers` Dense layers of `features` (64, 128 or 256) outputs, each followed
+ * by LayerNorm where gammas is not NULL (256 features) and the activation (SiLU
+ * with LayerNorm only); the actor head of A outputs and the value head; the
+ * categorical draw (scale NULL, action int32 [rows]) or the Gaussian one (raw
+ * scale [A], action float [rows, A]).  weights / biases / gammas / betas: HOST
+ * arrays of 2 * layers device pointers, the actor's layers, then the critic's
+ * (16-byte aligned, kernels [K_l, features]; a bias may be NULL); head_w / ldwh
+ * / head_b: 2 entries each.  Same outputs as the layer-by-layer GEMMs, the head
+ * GEMMs and the sampling launch. */
+int ppo_step_towers_max_layers(void);
+int ppo_step_towers_max_outputs(void);
+int ppo_step_towers_f32(void* stream, const float* obs, int64_t ldo, int rows, int obs_dim, int layers, int features,
+                        const float* const* weights, const float* const* biases, const float* const* gammas,
+                        const float* const* betas, float eps, int act, const float* const* head_w, const int64_t* ldwh,
+                        const float* const* head_b, int A, const float* scale, const uint32_t* key, float temperature,
+                        void* action, float* log_prob, float* value);
+
 /* --------------------------------------------- prioritised env selection
  * Replaces the minibatch selection of RecurrentPuPO.update
  * (boonta/algorithms/recurrent_pupo.py:226-236): priority[n] =
