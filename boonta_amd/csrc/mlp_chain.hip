@@ -711,11 +711,15 @@ __global__ void __launch_bounds__(MC_THREADS) mlp_ln_fwd_bwd_kernel(FwdArgs p, H
 // where its own lane wrote them, so there are no statistics and no transposed
 // kernels: dX = dZ W^T reads W along its rows (64-byte pieces), one contraction
 // per inner layer.  What bounds it: every workgroup streams the kernels from L2
-// for 16 rows (about 40 bytes a clock per CU) beside their fp32 MFMAs, 6-7 us a
-// 256 x 256 contraction (8 and 16 waves a workgroup were no faster, 38 and 56 us
-// against 37), and for small towers latency.  2 x 256 tanh towers over 2048 rows
-// of 87 inputs: seven launches of 72 us before, one of 37; 2 x 64 towers over
-// 128 rows of 4: 46 us, 11 (four waves; 128 wide on eight: 17.1 us, on four 18.4).
+// for 16 rows beside their fp32 MFMAs, and the optimizer step before has left
+// none of them there, so from 32 row blocks on the blocks of an XCD first bring
+// their tower's kernels in together (warm_l2; with fewer a block would fetch
+// most of a kernel that it reads itself anyway).  That takes a 2 x 256 tanh
+// update of 32 minibatches of 2048 rows from 2247 to 2155 us, and eight waves
+// then beat four: 2113 (before it they were no faster).  2 x 256 tanh towers over
+// 2048 rows of 87 inputs: seven launches of 72 us, then one of 37, now about 33;
+// 2 x 64 towers over 128 rows of 4: 46 us, 11 (four waves; 128 wide on eight:
+// 17.1 us, on four 18.4).
 struct ActArgs {
   const float* X;  // layer 0 input rows (row r is X[idx[r]] when idx is non-null)
   int64_t ldx;
@@ -782,6 +786,7 @@ __global__ void __launch_bounds__(64 * NW) mlp_act_kernel(ActArgs p, HeadLossPar
   __shared__ double s_st[MC_ROWS][NSTAT];
   __shared__ float s_dsc[MC_ROWS][16];
   __shared__ __attribute__((aligned(1024))) float s_hk[F * 16];  // the tower's head kernel
+  __shared__ __attribute__((aligned(1024))) float s_warm[256 * NW];
   const int64_t t = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -797,6 +802,8 @@ __global__ void __launch_bounds__(64 * NW) mlp_act_kernel(ActArgs p, HeadLossPar
     lane_samples(hp, r0, threadIdx.x, lin);
     copy_head_w<HB>(hp, t == 0, s_hk);
   }
+  if (gridDim.x >= 32)  // (at least four blocks of a tower per XCD)
+    for (int l = 0; l < p.L; ++l) warm_l2<NW>(p.W[l] + t * p.tP, (l ? F : p.K0) * F, s_warm);
 
   for (int l = 0; l < p.L; ++l) {
     if (wave < 4 && l == p.L - 1) lane_gathers(hp, threadIdx.x & 15, lin);
@@ -827,7 +834,7 @@ __global__ void __launch_bounds__(64 * NW) mlp_act_kernel(ActArgs p, HeadLossPar
   }
 
   // heads and loss; the last layer's dZ goes to memory and into the tile (the
-  // head kernel's copies, issued first, are long complete)
+  // copies into LDS, issued first, are long complete)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (wave < 4) {
@@ -1161,7 +1168,7 @@ PPO_EXPORT int ppo_mlp_act_fwd_head_loss_bwd_f32(
 #define PPO_ACT_CHAIN_W(ACTV)                         \
   if (F == 64) { PPO_ACT_CHAIN(64, 4, ACTV) }         \
   else if (F == 128) { PPO_ACT_CHAIN(128, 8, ACTV) }  \
-  else { PPO_ACT_CHAIN(256, 4, ACTV) }
+  else { PPO_ACT_CHAIN(256, 8, ACTV) }
   switch (act) {
     case ACT_RELU: PPO_ACT_CHAIN_W(ACT_RELU) break;
     case ACT_TANH: PPO_ACT_CHAIN_W(ACT_TANH) break;

@@ -94,4 +94,16 @@ __device__ __forceinline__ void act_contract(floatx4 (&acc)[NB], const float* ar
   }
 }
 
+// Brings this workgroup's share of n floats at p into the L2 of its XCD with
+// copies into the wave's 1 KB of scratch LDS (256-float pieces; a remainder is
+// left out): workgroups go to the 8 XCDs in turn, so blocks x, x + 8, .. of a
+// tower share one L2.  Wait for the copies before the LDS is used or freed.
+template <int NW>
+__device__ __forceinline__ void warm_l2(const float* p, int n, float* scratch) {
+  const int wave = threadIdx.x >> 6;
+  const int share = blockIdx.x >> 3, shares = (gridDim.x + 7) >> 3;
+  for (int c = share * NW + wave; c < n / 256; c += shares * NW)
+    ppo::lds_copy16(p + 256 * c + 4 * (threadIdx.x & 63), scratch + 256 * wave);
+}
+
 }  // namespace
