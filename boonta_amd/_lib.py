@@ -52,6 +52,8 @@ SIGNATURES = {
     "ppo_step_towers_max_layers": (I, []),
     "ppo_step_towers_max_outputs": (I, []),
     "ppo_step_towers_f32": (I, [P, P, I64, I, I, I, I, P, P, P, P, F, I, P, P, P, I, P, P, F, P, P, P]),
+    "ppo_head_sample_categorical_f32": (I, [P, P, I64, I, I, P, I64, P, I, P, F, P, P, P]),
+    "ppo_gru_fwd_step_x_f32": (I, [P, P, I64, I, P, I64, P, P, I64, P, P, P, I64, P, P, I64, I, I]),
     "ppo_priority_choice_max_envs": (I, []),
     "ppo_priority_choice_f32": (I, [P, P, I64, I, I, F, F, P, I, P, P, P]),
     "ppo_gemm_ln_act_fwd_f32": (I, [P, P, I64, P, P, I64, P, P, P, P, I64, P, I64, P, P, I, I, I, F, I]),

@@ -87,15 +87,24 @@ struct FwdArgs {
   float* hp_out; int64_t ldhp;
   float* gates; int64_t ldg;
   int Bm, H;
+  // XW: the input projections formed here, x [Bm, I] wi [I, 3H] + bi (xi unused)
+  const float* x; int64_t ldx;
+  const float* wi; int64_t ldwi;
+  const float* bi;
+  int I;
 };
 
 // grid (ceil(Bm / 16), H / 16), block 256.  NIT: 16-wide k steps per wave
 // (H / 64) when known at compile time (all of a wave's loads then issue
 // before its first MFMA); 0: a runtime loop.  The epilogue's operands are
-// loaded at entry, so their latency overlaps the contraction's.
-template <int NIT>
+// loaded at entry, so their latency overlaps the contraction's.  XW: the
+// tile's input projections are a second contraction here, over x's I features
+// (I == H when NIT > 0): one step needs its own 16 x 48 of them once, so a GEMM
+// ahead costs a launch and a round trip of [Bm, 3H] for nothing.
+template <int NIT, bool XW = false>
 __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
   __shared__ float red[WAVES][3][TILE][TILE + 1];
+  __shared__ float redx[XW ? WAVES : 1][3][TILE][TILE + 1];
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
@@ -124,9 +133,30 @@ __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
       for (int g = 0; g < 3; ++g) bv[g][s] = wr[g * H];
     }
   };
+  // x's row and the columns u0 + i of the (in, ir, iz) blocks of wi
+  const float* xrow = XW ? a.x + (int64_t)bc * a.ldx : nullptr;
+  const float* xcol = XW ? a.wi + u0 + i : nullptr;
+  const int xspan = XW ? a.I / WAVES : 0;
+  const int xbeg = wave * xspan;
+  auto load_x = [&](int base, floatx4& av, float (&bv)[3][4]) {
+    const int k = base + 4 * kq;
+    av = *reinterpret_cast<const floatx4*>(xrow + k);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float* wr = xcol + (int64_t)(k + s) * a.ldwi;
+#pragma unroll
+      for (int g = 0; g < 3; ++g) bv[g][s] = wr[g * H];
+    }
+  };
   floatx4 av[NIT > 0 ? NIT : 1];
   float bv[NIT > 0 ? NIT : 1][3][4];
+  floatx4 xv[XW && NIT > 0 ? NIT : 1];
+  float wv[XW && NIT > 0 ? NIT : 1][3][4];
   if (NIT > 0) {
+    if constexpr (XW) {
+#pragma unroll
+      for (int it = 0; it < NIT; ++it) load_x(xbeg + 16 * it, xv[it], wv[it]);
+    }
 #pragma unroll
     for (int it = 0; it < NIT; ++it) load(kbeg + 16 * it, av[it], bv[it]);
   }
@@ -139,17 +169,36 @@ __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
   const int u = u0 + tj;
   const bool bb_ok = bb < a.Bm;
   const int bbc = bb_ok ? bb : b0;
-  const float* x = a.xi + (int64_t)bbc * a.ldxi;
-  const float xn = x[u], xr = x[H + u], xz = x[2 * H + u];
+  const float* x = XW ? a.bi : a.xi + (int64_t)bbc * a.ldxi;
+  float xn = x[u], xr = x[H + u], xz = x[2 * H + u];
   const float bhn = a.bhn[u];
   const bool reset_e = bb_ok ? done_at(a.term, a.trunc, a.flag_rows, bb) : true;
   const int64_t re = a.hprev_rows ? (int64_t)a.hprev_rows[bbc] : (int64_t)bbc;
   const float hp_raw = a.hprev[re * a.ldh + u];
   issue_fence();
 
-  floatx4 acc[3];
+  floatx4 acc[3], accx[3];  // accx: columns (in, ir, iz)
 #pragma unroll
-  for (int g = 0; g < 3; ++g) acc[g] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int g = 0; g < 3; ++g) acc[g] = accx[g] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (XW) {
+    auto mma_x = [&](floatx4 avv, const float (&bvv)[3][4]) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int g = 0; g < 3; ++g) accx[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(avv[s], bvv[g][s], accx[g], 0, 0, 0);
+    };
+    if constexpr (NIT > 0) {
+#pragma unroll
+      for (int it = 0; it < NIT; ++it) mma_x(xv[it], wv[it]);
+    } else {
+      for (int base = xbeg; base < xbeg + xspan; base += 16) {
+        floatx4 a1;
+        float b1[3][4];
+        load_x(base, a1, b1);
+        mma_x(a1, b1);
+      }
+    }
+  }
   auto mma = [&](floatx4 avv, const float (&bvv)[3][4]) {
     if (!live) avv = floatx4{0.f, 0.f, 0.f, 0.f};  // a reset sequence starts from h = 0
 #pragma unroll
@@ -173,10 +222,23 @@ __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
 #pragma unroll
   for (int g = 0; g < 3; ++g)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) red[wave][g][4 * kq + v][i] = acc[g][v];
+    for (int v = 0; v < 4; ++v) {
+      red[wave][g][4 * kq + v][i] = acc[g][v];
+      if constexpr (XW) redx[wave][g][4 * kq + v][i] = accx[g][v];
+    }
   __syncthreads();
 
   if (!bb_ok) return;
+  if constexpr (XW) {
+    float s[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+#pragma unroll
+      for (int g = 0; g < 3; ++g) s[g] += redx[w][g][ti][tj];
+    xn += s[0];
+    xr += s[1];
+    xz += s[2];
+  }
   float ar = 0.f, az = 0.f, an = 0.f;
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) {
@@ -1012,7 +1074,7 @@ PPO_EXPORT int ppo_gru_fwd_step_f32(void* stream, const float* xi, int64_t ldxi,
   if (!aligned16(hprev) || ldh % 4 != 0)
     return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_f32: hprev rows must be 16-byte aligned");
   FwdArgs a{xi, ldxi, hprev, ldh, hprev_rows, terminated, truncated, flag_rows, wh, ldwh, bhn,
-            h_out, ldo, hp_out, ldhp, gates, ldg, Bm, H};
+            h_out, ldo, hp_out, ldhp, gates, ldg, Bm, H, nullptr, 0, nullptr, 0, nullptr, 0};
   dim3 grid(ppo::ceil_div(Bm, TILE), H / TILE);
   hipStream_t st = ppo::as_stream(stream);
   switch (H / 64) {  // 16-wide k steps per wave
@@ -1023,6 +1085,33 @@ PPO_EXPORT int ppo_gru_fwd_step_f32(void* stream, const float* xi, int64_t ldxi,
     default: hipLaunchKernelGGL(gru_fwd_step_kernel<0>, grid, dim3(256), 0, st, a); break;
   }
   return ppo::check_launch("ppo_gru_fwd_step_f32");
+}
+
+PPO_EXPORT int ppo_gru_fwd_step_x_f32(void* stream, const float* x, int64_t ldx, int I, const float* wi, int64_t ldwi,
+                                      const float* bi, const float* hprev, int64_t ldh, const uint8_t* terminated,
+                                      const uint8_t* truncated, const float* wh, int64_t ldwh, const float* bhn,
+                                      float* h_out, int64_t ldo, int Bm, int H) {
+  if (Bm < 0 || H <= 0 || H % 64 != 0 || I <= 0 || I % 64 != 0)
+    return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_x_f32: need Bm >= 0, H and I positive multiples of 64 "
+                          "(Bm=%d H=%d I=%d)", Bm, H, I);
+  if (Bm == 0) return PPO_OK;
+  if (!x || !wi || !bi || !hprev || !wh || !bhn || !h_out)
+    return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_x_f32: null buffer");
+  if (ldx < I || ldwi < 3 * H || ldh < H || ldwh < 3 * H || ldo < H)
+    return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_x_f32: leading dimension too small");
+  if (!aligned16(hprev) || ldh % 4 != 0 || !aligned16(x) || ldx % 4 != 0)
+    return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_x_f32: x and hprev rows must be 16-byte aligned");
+  FwdArgs a{nullptr, 0, hprev, ldh, nullptr, terminated, truncated, nullptr, wh, ldwh, bhn,
+            h_out, ldo, nullptr, 0, nullptr, 0, Bm, H, x, ldx, wi, ldwi, bi, I};
+  dim3 grid(ppo::ceil_div(Bm, TILE), H / TILE);
+  hipStream_t st = ppo::as_stream(stream);
+  switch (I == H ? H / 64 : 0) {  // 16-wide k steps per wave of both contractions
+    case 1: hipLaunchKernelGGL((gru_fwd_step_kernel<1, true>), grid, dim3(256), 0, st, a); break;
+    case 2: hipLaunchKernelGGL((gru_fwd_step_kernel<2, true>), grid, dim3(256), 0, st, a); break;
+    case 4: hipLaunchKernelGGL((gru_fwd_step_kernel<4, true>), grid, dim3(256), 0, st, a); break;
+    default: hipLaunchKernelGGL((gru_fwd_step_kernel<0, true>), grid, dim3(256), 0, st, a); break;
+  }
+  return ppo::check_launch("ppo_gru_fwd_step_x_f32");
 }
 
 PPO_EXPORT int ppo_gru_bwd_step_f32(void* stream, const float* dg, int64_t lddg, const float* wh, int64_t ldwh,

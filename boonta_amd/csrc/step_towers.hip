@@ -191,6 +191,77 @@ __global__ void __launch_bounds__(64 * NW, F == 256 ? 4 : 1) step_towers_kernel(
   }
 }
 
+// A shared head of at most 16 outputs and its categorical draw: 16 rows per
+// workgroup, the contraction over the F features split over eight waves (alternate
+// 16-deep chunks), then a 16-lane group per row.  Bound by latency; instead of
+// the head GEMM, whose 64-column tiles are three quarters padding, and the
+// sampling launch.
+constexpr int HS_WAVES = 8;
+
+struct HeadSampleArgs {
+  const float* X;  // [rows, F]
+  int64_t ldx;
+  int rows, F;
+  const float* Wh;  // [F, ldwh]: A logits, then the value
+  int64_t ldwh;
+  const float* bh;
+  int A;
+  const uint32_t* key;
+  float temperature;
+  int32_t* action;
+  float* log_prob;
+  float* value;
+};
+
+__global__ void __launch_bounds__(64 * HS_WAVES) head_sample_kernel(HeadSampleArgs p) {
+  __shared__ float s_head[HS_WAVES][ST_ROWS][ST_HEAD + 1];
+  __shared__ float s_out[ST_ROWS][ST_HEAD + 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15;
+  const int kq = lane >> 4;
+  const int r0 = blockIdx.x * ST_ROWS;
+  const bool a_live = r0 + li < p.rows;
+  const float* xrow = p.X + (int64_t)(a_live ? r0 + li : r0) * p.ldx;
+  const bool out_live = li <= p.A;
+  const float* wcol = p.Wh + (out_live ? li : 0);
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k0 = 16 * wave; k0 < p.F; k0 += 16 * HS_WAVES) {
+    const int k = k0 + 4 * kq;
+    const floatx4 x = *reinterpret_cast<const floatx4*>(xrow + k);
+    float w[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) w[s] = wcol[(k + s) * p.ldwh];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a_live ? x[s] : 0.f, out_live ? w[s] : 0.f, acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) s_head[wave][4 * kq + v][li] = acc[v];
+  __syncthreads();
+  const int row = threadIdx.x / 16;
+  const int j0 = threadIdx.x % 16;
+  const int r = r0 + row;
+  if (wave < 4) {
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < HS_WAVES; w += 2) o += s_head[w][row][j0] + s_head[w + 1][row][j0];
+    s_out[row][j0] = o + (j0 <= p.A && p.bh ? p.bh[j0] : 0.f);
+  }
+  __syncthreads();
+  if (wave >= 4) return;
+  const bool row_ok = r < p.rows;
+  int act_i;
+  float lp;
+  ppo::cat::draw(&s_out[row][0], p.A, row_ok, r, p.key[0], p.key[1], p.temperature, j0, act_i, lp);
+  if (row_ok && j0 == 0) {
+    p.action[r] = act_i;
+    p.log_prob[r] = lp;
+    p.value[r] = s_out[row][p.A];
+  }
+}
+
 bool aligned16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
 
 }  // namespace
@@ -210,8 +281,8 @@ PPO_EXPORT int ppo_step_towers_f32(void* stream, const float* obs, int64_t ldo, 
   if (rows < 0 || obs_dim < 1 || ldo < obs_dim || layers < 1 || layers > ST_MAX_LAYERS || act < 0 || act > 3 ||
       (F != 64 && F != 128 && F != 256) || (ln && (F != 256 || !betas)) || (!ln && act == ACT_SILU) ||
       (int64_t)obs_dim * F > INT32_MAX || A < 1 || A > ST_HEAD || !weights || !biases || !head_w || !ldwh || !head_b)
-    return ppo::set_error(PPO_ERR_ARG, "%s: bad argument (rows %d obs %d layers %d features %d act %d A %d)", name, rows,
-                          obs_dim, layers, F, act, A);
+    return ppo::set_error(PPO_ERR_ARG, "%s: bad argument (rows %d obs %d layers %d features %d act %d A %d)", name,
+                          rows, obs_dim, layers, F, act, A);
   if (rows == 0) return PPO_OK;
   if (!obs || !key || !action || !log_prob || !value) return ppo::set_error(PPO_ERR_ARG, "%s: null buffer", name);
   StepTowersArgs a{};
@@ -251,5 +322,21 @@ PPO_EXPORT int ppo_step_towers_f32(void* stream, const float* obs, int64_t ldo, 
   }
 #undef PPO_STEP_TOWERS_W
 #undef PPO_STEP_TOWERS
+  return ppo::check_launch(name);
+}
+
+PPO_EXPORT int ppo_head_sample_categorical_f32(void* stream, const float* x, int64_t ldx, int rows, int F,
+                                               const float* head_w, int64_t ldwh, const float* head_b, int A,
+                                               const uint32_t* key, float temperature, int32_t* action,
+                                               float* log_prob, float* value) {
+  const char* name = "ppo_head_sample_categorical_f32";
+  if (rows < 0 || F < 16 || F % 16 || ldx < F || ldx % 4 || A < 1 || A + 1 > ST_HEAD || ldwh < A + 1)
+    return ppo::set_error(PPO_ERR_ARG, "%s: bad argument (rows %d features %d A %d)", name, rows, F, A);
+  if (rows == 0) return PPO_OK;
+  if (!x || !head_w || !key || !action || !log_prob || !value || !aligned16(x))
+    return ppo::set_error(PPO_ERR_ARG, "%s: null or misaligned buffer", name);
+  HeadSampleArgs a{x, ldx, rows, F, head_w, ldwh, head_b, A, key, temperature, action, log_prob, value};
+  hipLaunchKernelGGL(head_sample_kernel, dim3(ppo::ceil_div(rows, ST_ROWS)), dim3(64 * HS_WAVES), 0,
+                     ppo::as_stream(stream), a);
   return ppo::check_launch(name);
 }

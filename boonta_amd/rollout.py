@@ -31,6 +31,16 @@ from .learner import (A_ROW, B_KN, EPI_BIAS_ACT, LayerBufs, DenseSpec, FlatState
                       split_forward_bufs)
 
 
+def _head_samples(program: Program, lib) -> bool:
+    """Whether ppo_head_sample_categorical_f32 takes the program's shared head:
+    on a trunk's float32 features (the executor's own, 16-byte rows) at every
+    number of rows."""
+    h = program.head_a
+    return (not program.bf16 and program.shared_head and bool(program.trunk) and program.dist["kind"] == "categorical"
+            and program.head_out == program.dist["num"] and program.head_out + 1 <= lib.ppo_step_towers_max_outputs()
+            and h.fin % 16 == 0)
+
+
 class StepExecutor(ForwardChain):
     """PPO.step for a fixed number of environments (rows).
 
@@ -66,6 +76,8 @@ class StepExecutor(ForwardChain):
             self.HC = torch.zeros(rows, hc.w.ld, **f32)
         self.KEY = torch.zeros(2, dtype=torch.int32, device=dev)
         self.fused = fused and self._fusable(lib)
+        self.head_samples = fused and _head_samples(program, lib)
+        self.trunk_tables = self._trunk_tables() if self.fused else None
         self.towers = self._tower_tables() if fused and self._towers_fusable(lib) else None
 
     def _fusable(self, lib) -> bool:
@@ -82,6 +94,15 @@ class StepExecutor(ForwardChain):
         h = prog.head_a
         return h.fin == 256 and h.w.ld <= 16 and prog.head_out == prog.dist["num"] and prog.head_out + 1 <= h.w.ld
 
+    def _trunk_tables(self) -> dict:
+        """Host arrays of ppo_step_mlp_categorical_f32's parameter pointers."""
+        prog, view, h = self.prog, self.flat.view, self.prog.head_a
+        n = len(prog.trunk)
+        keep = ((ctypes.c_void_p * n)(*[view(s.dense.w) for s in prog.trunk]),
+                (ctypes.c_int64 * n)(*[s.ld for s in prog.trunk]),
+                (ctypes.c_void_p * n)(*[view(s.dense.b) if s.dense.b is not None else None for s in prog.trunk]))
+        return {"keep": keep, "args": (n, *map(ctypes.addressof, keep), _act(prog.trunk[0].act), view(h.w), h.w.ld)}
+
     def _towers_fusable(self, lib) -> bool:
         """Whether the paired towers' one-launch step covers this program: for
         every number of rows it replaces two launches per layer and three after
@@ -93,7 +114,8 @@ class StepExecutor(ForwardChain):
             return False
         s0 = A[0]
         F, ln = s0.fout, s0.ln is not None
-        if F not in ((256,) if ln else (64, 128, 256)) or s0.act not in ("relu", "tanh", None) + (("silu",) if ln else ()):
+        if (F not in ((256,) if ln else (64, 128, 256))
+                or s0.act not in ("relu", "tanh", None) + (("silu",) if ln else ())):
             return False
         for layers in (A, C):
             for i, s in enumerate(layers):
@@ -150,13 +172,8 @@ class StepExecutor(ForwardChain):
         prog = self.prog
         rows = self.rows
         if self.fused:
-            h, n = prog.head_a, len(prog.trunk)
-            # host arrays of the trunk's kernel / bias pointers (read at launch)
-            ws = (ctypes.c_void_p * n)(*[self.flat.view(s.dense.w) for s in prog.trunk])
-            lds = (ctypes.c_int64 * n)(*[s.ld for s in prog.trunk])
-            bs = (ctypes.c_void_p * n)(*[self.flat.view(s.dense.b) if s.dense.b is not None else None
-                                         for s in prog.trunk])
-            self._call("ppo_step_mlp_categorical_f32", st, obs, ldo, rows, prog.trunk[0].dense.fin, n, ws, lds, bs, _act(prog.trunk[0].act), self.flat.view(h.w), h.w.ld,
+            h, t = prog.head_a, self.trunk_tables
+            self._call("ppo_step_mlp_categorical_f32", st, obs, ldo, rows, prog.trunk[0].dense.fin, *t["args"],
                        self.flat.view(h.b) if h.b is not None else None, prog.dist["num"], key, float(temperature),
                        action, log_prob, value)
             return
@@ -166,6 +183,12 @@ class StepExecutor(ForwardChain):
             return
         if prog.shared_head:
             x, ldx, _ = self._fwd_layers(st, self.trunk, obs, ldo, None, rows)
+            if self.head_samples:
+                h = prog.head_a
+                self._call("ppo_head_sample_categorical_f32", st, x, ldx, rows, h.fin, self.flat.view(h.w), h.w.ld,
+                           self.flat.view(h.b) if h.b is not None else None, prog.head_out, key, float(temperature),
+                           action, log_prob, value)
+                return
             self._head(st, x, ldx, prog.head_a, self.HEAD)
             head, ldh = self.HEAD, self.HEAD.shape[1]
             vsrc, ldv = _p(self.HEAD) + 4 * prog.head_out, ldh
@@ -204,9 +227,17 @@ class StepExecutor(ForwardChain):
 class RecurrentStepExecutor(ForwardChain):
     """RecurrentPPO.step for a fixed number of environments (rows): the
     network of ``Network(feature_extractor=<MLP>, torso=RNN(GRUCell(H)),
-    head=ActorCritic(Dense, Dense))`` one time step at a time."""
+    head=ActorCritic(Dense, Dense))`` one time step at a time: the trunk's
+    launches, one for the GRU step with its input projections (a trunk width that
+    is a multiple of 64), one for the head and the draw (at most 15 logits);
+    ``fused=False`` issues the projection GEMM, the head GEMM and the sampling
+    launch instead (128 -> 256 -> GRU 256, 1024 envs: 43 -> 31
+    us a step, a key copy left out besides)."""
 
-    def __init__(self, program: Program, flat: FlatState, rows: int):
+    def __init__(self, program: Program, flat: FlatState, rows: int, fused: bool | None = None):
+        # (None: fused where the parameters are on the device, not where launches
+        # are recorded over host memory)
+        fused = flat.P.is_cuda if fused is None else fused
         if program.gru is None:
             raise TypeError("RecurrentStepExecutor needs a program with a GRU torso")
         if not program.shared_head or not program.trunk:
@@ -223,7 +254,10 @@ class RecurrentStepExecutor(ForwardChain):
         f32 = dict(dtype=torch.float32, device=dev)
         self.rows = rows
         self.trunk: list[LayerBufs] = [forward_bufs(s, rows, dev) for s in program.trunk]
-        self.XI = torch.zeros(rows, 3 * H, **f32)
+        self.input_proj = fused and program.gru.fin % 64 == 0
+        self.head_samples = fused and _head_samples(program, lib)
+        if not self.input_proj:
+            self.XI = torch.zeros(rows, 3 * H, **f32)
         self.HEAD = torch.zeros(rows, program.head_a.w.ld, **f32)
         self.KEY = torch.zeros(2, dtype=torch.int32, device=dev)
 
@@ -238,11 +272,21 @@ class RecurrentStepExecutor(ForwardChain):
         H, I = g.H, g.fin
         rows = self.rows
         x, ldx, _ = self._fwd_layers(st, self.trunk, obs, ldo, None, rows)
-        self._gemm(st, A_ROW, B_KN, x, ldx, None, self.flat.view(g.wi), 3 * H, _p(self.XI), 3 * H, rows, 3 * H, I,
-                   1, 0, EPI_BIAS_ACT, self.flat.view(g.bi), 0, None, None, 0, None, -1)
-        self._call("ppo_gru_fwd_step_f32", st, _p(self.XI), 3 * H, carry, H, None, terminated, truncated, None,
-                   self.flat.view(g.wh), 3 * H, self.flat.view(g.bhn), carry_out, H, None, H, None, 4 * H, rows, H)
+        if self.input_proj:
+            self._call("ppo_gru_fwd_step_x_f32", st, x, ldx, I, self.flat.view(g.wi), 3 * H, self.flat.view(g.bi),
+                       carry, H, terminated, truncated, self.flat.view(g.wh), 3 * H, self.flat.view(g.bhn), carry_out,
+                       H, rows, H)
+        else:
+            self._gemm(st, A_ROW, B_KN, x, ldx, None, self.flat.view(g.wi), 3 * H, _p(self.XI), 3 * H, rows, 3 * H, I,
+                       1, 0, EPI_BIAS_ACT, self.flat.view(g.bi), 0, None, None, 0, None, -1)
+            self._call("ppo_gru_fwd_step_f32", st, _p(self.XI), 3 * H, carry, H, None, terminated, truncated, None,
+                       self.flat.view(g.wh), 3 * H, self.flat.view(g.bhn), carry_out, H, None, H, None, 4 * H, rows, H)
         h = prog.head_a
+        if self.head_samples:
+            self._call("ppo_head_sample_categorical_f32", st, carry_out, H, rows, H, self.flat.view(h.w), h.w.ld,
+                       self.flat.view(h.b) if h.b is not None else None, prog.head_out, key, float(temperature),
+                       action, log_prob, value)
+            return
         self._gemm(st, A_ROW, B_KN, carry_out, H, None, self.flat.view(h.w), h.w.ld, _p(self.HEAD), h.w.ld, rows,
                    h.w.ld, h.fin, 1, 0, EPI_BIAS_ACT, self.flat.view(h.b) if h.b is not None else None, 0, None,
                    None, 0, None, -1)

@@ -175,6 +175,13 @@ int ppo_step_towers_f32(void* stream, const float* obs, int64_t ldo, int rows, i
                         const float* const* head_b, int A, const float* scale, const uint32_t* key, float temperature,
                         void* action, float* log_prob, float* value);
 
+/* A shared head of A logits and the value (A + 1 <= ppo_step_towers_max_outputs())
+ * on the features x [rows, ldx] (16-byte rows, F a multiple of 16), and the draw
+ * of ppo_sample_categorical_f32, in one launch. */
+int ppo_head_sample_categorical_f32(void* stream, const float* x, int64_t ldx, int rows, int F, const float* head_w,
+                                    int64_t ldwh, const float* head_b, int A, const uint32_t* key, float temperature,
+                                    int32_t* action, float* log_prob, float* value);
+
 /* --------------------------------------------- prioritised env selection
  * Replaces the minibatch selection of RecurrentPuPO.update
  * (boonta/algorithms/recurrent_pupo.py:226-236): priority[n] =
@@ -710,6 +717,13 @@ int ppo_gru_fwd_step_f32(void* stream, const float* xi, int64_t ldxi, const floa
                          const int32_t* hprev_rows, const uint8_t* terminated, const uint8_t* truncated,
                          const int32_t* flag_rows, const float* wh, int64_t ldwh, const float* bhn, float* h_out,
                          int64_t ldo, float* hp_out, int64_t ldhp, float* gates, int64_t ldg, int Bm, int H);
+/* The same step from the input features x [Bm, I] (I a multiple of 64, 16-byte
+ * rows): the projections x wi + bi (wi [I, 3H], columns (in, ir, iz)) are formed
+ * in the launch; nothing is kept for a backward. */
+int ppo_gru_fwd_step_x_f32(void* stream, const float* x, int64_t ldx, int I, const float* wi, int64_t ldwi,
+                           const float* bi, const float* hprev, int64_t ldh, const uint8_t* terminated,
+                           const uint8_t* truncated, const float* wh, int64_t ldwh, const float* bhn, float* h_out,
+                           int64_t ldo, int Bm, int H);
 int ppo_gru_bwd_step_f32(void* stream, const float* dg, int64_t lddg, const float* wh, int64_t ldwh,
                          const float* dh_t, int64_t lddht, const float* z_t, int64_t ldz, const uint8_t* terminated,
                          const uint8_t* truncated, const int32_t* flag_rows, const float* dout, int64_t lddo,
