@@ -76,14 +76,14 @@ class RecurrentPPO(PPO):
         for name in ("terminated", "truncated"):
             f = getattr(timestep, name)
             flags.append(None if f is None else self._need(f, torch.bool, f"timestep.{name}", (N,)))
-        self._set_key(ex, key)
+        key_ptr = self._key_pointer(ex, key)
         new_carry = torch.empty(N, H, dtype=torch.float32, device=dev)
         action = torch.empty(N, dtype=torch.int32, device=dev)
         log_prob = torch.empty(N, dtype=torch.float32, device=dev)
         value = torch.empty(N, dtype=torch.float32, device=dev)
         ex.issue(torch.cuda.current_stream().cuda_stream, obs.data_ptr(), obs_dim, carry.data_ptr(), flags[0],
                  flags[1], float(temperature), new_carry.data_ptr(), action.data_ptr(), log_prob.data_ptr(),
-                 value.data_ptr())
+                 value.data_ptr(), key=key_ptr)
         return state, new_carry, action, {"log_prob": log_prob, "value": value}
 
     def update(self, state, key, transitions):
