@@ -157,6 +157,20 @@ def _single_launch_work(name, args):
         rows, K0, L, ldwh = args[3], args[4], args[5], args[11]
         weights = K0 * 256 + (L - 1) * 256 * 256 + 256 * ldwh
         return 2.0 * rows * weights, 4.0 * (rows * K0 + weights + 3 * rows)
+    if name == "ppo_step_towers_f32":
+        rows, K0, L, F, A = args[3], args[4], args[5], args[6], args[16]
+        weights = 2 * (K0 * F + (L - 1) * F * F) + F * (A + 1)
+        return 2.0 * rows * weights, 4.0 * (rows * (K0 + A + 2) + weights)
+    if name == "ppo_head_sample_categorical_f32":
+        rows, F, A = args[3], args[4], args[8]
+        return 2.0 * rows * F * (A + 1), 4.0 * (rows * (F + 3) + F * (A + 1))
+    if name == "ppo_gru_fwd_step_x_f32":
+        I, Bm, H = args[3], args[-2], args[-1]
+        return 2.0 * Bm * 3 * H * (H + I), 4.0 * (Bm * (I + 2 * H) + 3 * H * (H + I))
+    if name == "ppo_mlp_act_fwd_head_loss_bwd_f32":
+        towers, L, M, K0, F = args[1], args[2], args[6], args[7], args[9]
+        inner = (L - 1) * F * F
+        return 2.0 * towers * M * (K0 * F + 2 * inner), 4.0 * (M * K0 + towers * (2 * M * L * F + K0 * F + inner))
     if name == "ppo_sample_categorical_f32":
         rows, A = args[3], args[4]
         return 0.0, 4.0 * rows * (A + 4)
@@ -296,6 +310,12 @@ def _single_launch_shape(name, args):
         return [args[15], args[17], args[16]]
     if name == "ppo_step_mlp_categorical_f32":
         return [args[3], 256, args[4], args[5]]
+    if name == "ppo_step_towers_f32":
+        return [args[3], args[6], args[4], args[5], 2]
+    if name == "ppo_head_sample_categorical_f32":
+        return [args[3], args[8] + 1, args[4]]
+    if name == "ppo_mlp_act_fwd_head_loss_bwd_f32":
+        return [args[6], args[9], args[7], args[2], args[1]]
     if name in ("ppo_mlp_ln_fwd_f32", "ppo_mlp_ln_fwd_head_loss_f32", "ppo_mlp_ln_fwd_head_loss_bwd_f32"):
         return [args[6], 256, args[7], args[2], args[1]]
     if name == "ppo_mlp_ln_bwd_f32":
