@@ -87,24 +87,15 @@ struct FwdArgs {
   float* hp_out; int64_t ldhp;
   float* gates; int64_t ldg;
   int Bm, H;
-  // XW: the input projections formed here, x [Bm, I] wi [I, 3H] + bi (xi unused)
-  const float* x; int64_t ldx;
-  const float* wi; int64_t ldwi;
-  const float* bi;
-  int I;
 };
 
 // grid (ceil(Bm / 16), H / 16), block 256.  NIT: 16-wide k steps per wave
 // (H / 64) when known at compile time (all of a wave's loads then issue
 // before its first MFMA); 0: a runtime loop.  The epilogue's operands are
-// loaded at entry, so their latency overlaps the contraction's.  XW: the
-// tile's input projections are a second contraction here, over x's I features
-// (I == H when NIT > 0): one step needs its own 16 x 48 of them once, so a GEMM
-// ahead costs a launch and a round trip of [Bm, 3H] for nothing.
-template <int NIT, bool XW = false>
+// loaded at entry, so their latency overlaps the contraction's.
+template <int NIT>
 __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
   __shared__ float red[WAVES][3][TILE][TILE + 1];
-  __shared__ float redx[XW ? WAVES : 1][3][TILE][TILE + 1];
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
@@ -133,30 +124,9 @@ __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
       for (int g = 0; g < 3; ++g) bv[g][s] = wr[g * H];
     }
   };
-  // x's row and the columns u0 + i of the (in, ir, iz) blocks of wi
-  const float* xrow = XW ? a.x + (int64_t)bc * a.ldx : nullptr;
-  const float* xcol = XW ? a.wi + u0 + i : nullptr;
-  const int xspan = XW ? a.I / WAVES : 0;
-  const int xbeg = wave * xspan;
-  auto load_x = [&](int base, floatx4& av, float (&bv)[3][4]) {
-    const int k = base + 4 * kq;
-    av = *reinterpret_cast<const floatx4*>(xrow + k);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const float* wr = xcol + (int64_t)(k + s) * a.ldwi;
-#pragma unroll
-      for (int g = 0; g < 3; ++g) bv[g][s] = wr[g * H];
-    }
-  };
   floatx4 av[NIT > 0 ? NIT : 1];
   float bv[NIT > 0 ? NIT : 1][3][4];
-  floatx4 xv[XW && NIT > 0 ? NIT : 1];
-  float wv[XW && NIT > 0 ? NIT : 1][3][4];
   if (NIT > 0) {
-    if constexpr (XW) {
-#pragma unroll
-      for (int it = 0; it < NIT; ++it) load_x(xbeg + 16 * it, xv[it], wv[it]);
-    }
 #pragma unroll
     for (int it = 0; it < NIT; ++it) load(kbeg + 16 * it, av[it], bv[it]);
   }
@@ -169,36 +139,17 @@ __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
   const int u = u0 + tj;
   const bool bb_ok = bb < a.Bm;
   const int bbc = bb_ok ? bb : b0;
-  const float* x = XW ? a.bi : a.xi + (int64_t)bbc * a.ldxi;
-  float xn = x[u], xr = x[H + u], xz = x[2 * H + u];
+  const float* x = a.xi + (int64_t)bbc * a.ldxi;
+  const float xn = x[u], xr = x[H + u], xz = x[2 * H + u];
   const float bhn = a.bhn[u];
   const bool reset_e = bb_ok ? done_at(a.term, a.trunc, a.flag_rows, bb) : true;
   const int64_t re = a.hprev_rows ? (int64_t)a.hprev_rows[bbc] : (int64_t)bbc;
   const float hp_raw = a.hprev[re * a.ldh + u];
   issue_fence();
 
-  floatx4 acc[3], accx[3];  // accx: columns (in, ir, iz)
+  floatx4 acc[3];
 #pragma unroll
-  for (int g = 0; g < 3; ++g) acc[g] = accx[g] = floatx4{0.f, 0.f, 0.f, 0.f};
-  if constexpr (XW) {
-    auto mma_x = [&](floatx4 avv, const float (&bvv)[3][4]) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int g = 0; g < 3; ++g) accx[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(avv[s], bvv[g][s], accx[g], 0, 0, 0);
-    };
-    if constexpr (NIT > 0) {
-#pragma unroll
-      for (int it = 0; it < NIT; ++it) mma_x(xv[it], wv[it]);
-    } else {
-      for (int base = xbeg; base < xbeg + xspan; base += 16) {
-        floatx4 a1;
-        float b1[3][4];
-        load_x(base, a1, b1);
-        mma_x(a1, b1);
-      }
-    }
-  }
+  for (int g = 0; g < 3; ++g) acc[g] = floatx4{0.f, 0.f, 0.f, 0.f};
   auto mma = [&](floatx4 avv, const float (&bvv)[3][4]) {
     if (!live) avv = floatx4{0.f, 0.f, 0.f, 0.f};  // a reset sequence starts from h = 0
 #pragma unroll
@@ -222,23 +173,10 @@ __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
 #pragma unroll
   for (int g = 0; g < 3; ++g)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      red[wave][g][4 * kq + v][i] = acc[g][v];
-      if constexpr (XW) redx[wave][g][4 * kq + v][i] = accx[g][v];
-    }
+    for (int v = 0; v < 4; ++v) red[wave][g][4 * kq + v][i] = acc[g][v];
   __syncthreads();
 
   if (!bb_ok) return;
-  if constexpr (XW) {
-    float s[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w)
-#pragma unroll
-      for (int g = 0; g < 3; ++g) s[g] += redx[w][g][ti][tj];
-    xn += s[0];
-    xr += s[1];
-    xz += s[2];
-  }
   float ar = 0.f, az = 0.f, an = 0.f;
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) {
@@ -257,6 +195,129 @@ __global__ void __launch_bounds__(256) gru_fwd_step_kernel(FwdArgs a) {
     g[H + u] = r;
     g[2 * H + u] = z;
     g[3 * H + u] = hn;
+  }
+}
+
+// One step from the input features: x [Bm, I], wi [I, 3H] + bi formed here
+// (columns in | ir | iz), with the recurrent contraction beside it; nothing kept
+// for a backward.  RT tiles of 16 sequences per workgroup share its 16 units'
+// columns of both kernels: with one tile each a step is bound by reading them
+// from L2 (1024 sequences of 256 -> 256: 100 MB, 19.9 us; four tiles 16.5).  NIT: 16-wide k steps
+// per wave of both contractions (I == H); 0: runtime loops.
+struct XStepArgs {
+  const float* x; int64_t ldx; int I;
+  const float* wi; int64_t ldwi;
+  const float* bi;
+  const float* hprev; int64_t ldh;
+  const uint8_t* term; const uint8_t* trunc;
+  const float* wh; int64_t ldwh;
+  const float* bhn;
+  float* h_out; int64_t ldo;
+  int Bm, H;
+};
+
+template <int NIT, int RT>
+__global__ void __launch_bounds__(256) gru_step_x_kernel(XStepArgs a) {
+  __shared__ float red[WAVES][6][TILE][TILE + 1];
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6;
+  const int lane = tid & 63;
+  const int i = lane & 15;
+  const int kq = lane >> 4;
+  const int b0 = blockIdx.x * TILE * RT;
+  const int u0 = blockIdx.y * TILE;
+  const int H = a.H;
+  // acc[rt][0..2]: x's (in, ir, iz) columns; [3..5]: h's (hr, hz, hn)
+  floatx4 acc[RT][6];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int g = 0; g < 6; ++g) acc[rt][g] = floatx4{0.f, 0.f, 0.f, 0.f};
+  bool live[RT];
+  int64_t row[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int b = b0 + 16 * rt + i;
+    row[rt] = min(b, a.Bm - 1);
+    live[rt] = b < a.Bm && !done_at(a.term, a.trunc, nullptr, b);
+  }
+  // one 16-deep piece of a contraction: A rows and the unit columns of W
+  auto load = [&](const float* A, int64_t lda, const float* W, int64_t ldw, int base, floatx4 (&av)[RT],
+                  float (&bv)[3][4]) {
+    const int k = base + 4 * kq;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) av[rt] = *reinterpret_cast<const floatx4*>(A + row[rt] * lda + k);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float* wr = W + (int64_t)(k + s) * ldw + u0 + i;
+#pragma unroll
+      for (int g = 0; g < 3; ++g) bv[g][s] = wr[g * H];
+    }
+  };
+  auto mma = [&](const floatx4 (&av)[RT], const float (&bv)[3][4], int g0) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const bool on = g0 == 0 || live[rt];  // a reset sequence starts from h = 0
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const float v = on ? av[rt][s] : 0.f;
+#pragma unroll
+        for (int g = 0; g < 3; ++g)
+          acc[rt][g0 + g] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, bv[g][s], acc[rt][g0 + g], 0, 0, 0);
+      }
+    }
+  };
+  if constexpr (NIT > 0) {
+    floatx4 xv[NIT][RT], hv[NIT][RT];
+    float xw[NIT][3][4], hw[NIT][3][4];
+    const int beg = wave * 16 * NIT;
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) load(a.x, a.ldx, a.wi, a.ldwi, beg + 16 * it, xv[it], xw[it]);
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) load(a.hprev, a.ldh, a.wh, a.ldwh, beg + 16 * it, hv[it], hw[it]);
+    issue_fence();
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) mma(xv[it], xw[it], 0);
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) mma(hv[it], hw[it], 3);
+  } else {
+    floatx4 av[RT];
+    float bv[3][4];
+    for (int k = wave * (a.I / WAVES); k < (wave + 1) * (a.I / WAVES); k += 16) {
+      load(a.x, a.ldx, a.wi, a.ldwi, k, av, bv);
+      mma(av, bv, 0);
+    }
+    for (int k = wave * (H / WAVES); k < (wave + 1) * (H / WAVES); k += 16) {
+      load(a.hprev, a.ldh, a.wh, a.ldwh, k, av, bv);
+      mma(av, bv, 3);
+    }
+  }
+  // per row tile: the waves' partial sums meet in LDS (lane: rows 4 kq + v,
+  // column i), one thread per (sequence, unit) finishes the cell
+  const int ti = tid >> 4;
+  const int tj = tid & 15;
+  const int u = u0 + tj;
+  const float bn = a.bi[u], br = a.bi[H + u], bz = a.bi[2 * H + u], bhn = a.bhn[u];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    if (rt) __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 6; ++g)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[wave][g][4 * kq + v][i] = acc[rt][g][v];
+    __syncthreads();
+    const int b = b0 + 16 * rt + ti;
+    if (b < a.Bm) {
+      float s[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w)
+#pragma unroll
+        for (int g = 0; g < 6; ++g) s[g] += red[w][g][ti][tj];
+      const float hp = done_at(a.term, a.trunc, nullptr, b) ? 0.f : a.hprev[(int64_t)b * a.ldh + u];
+      float r, z, hn, n;
+      a.h_out[(int64_t)b * a.ldo + u] =
+          gru_cell_fwd(br + s[1], s[3], bz + s[2], s[4], bn + s[0], s[5], bhn, hp, r, z, hn, n);
+    }
   }
 }
 
@@ -1074,7 +1135,7 @@ PPO_EXPORT int ppo_gru_fwd_step_f32(void* stream, const float* xi, int64_t ldxi,
   if (!aligned16(hprev) || ldh % 4 != 0)
     return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_f32: hprev rows must be 16-byte aligned");
   FwdArgs a{xi, ldxi, hprev, ldh, hprev_rows, terminated, truncated, flag_rows, wh, ldwh, bhn,
-            h_out, ldo, hp_out, ldhp, gates, ldg, Bm, H, nullptr, 0, nullptr, 0, nullptr, 0};
+            h_out, ldo, hp_out, ldhp, gates, ldg, Bm, H};
   dim3 grid(ppo::ceil_div(Bm, TILE), H / TILE);
   hipStream_t st = ppo::as_stream(stream);
   switch (H / 64) {  // 16-wide k steps per wave
@@ -1101,16 +1162,23 @@ PPO_EXPORT int ppo_gru_fwd_step_x_f32(void* stream, const float* x, int64_t ldx,
     return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_x_f32: leading dimension too small");
   if (!aligned16(hprev) || ldh % 4 != 0 || !aligned16(x) || ldx % 4 != 0)
     return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_x_f32: x and hprev rows must be 16-byte aligned");
-  FwdArgs a{nullptr, 0, hprev, ldh, nullptr, terminated, truncated, nullptr, wh, ldwh, bhn,
-            h_out, ldo, nullptr, 0, nullptr, 0, Bm, H, x, ldx, wi, ldwi, bi, I};
-  dim3 grid(ppo::ceil_div(Bm, TILE), H / TILE);
+  XStepArgs a{x, ldx, I, wi, ldwi, bi, hprev, ldh, terminated, truncated, wh, ldwh, bhn, h_out, ldo, Bm, H};
   hipStream_t st = ppo::as_stream(stream);
+  // the most row tiles per workgroup that leave one workgroup per CU
+  const int rt = ppo::ceil_div(Bm, 4 * TILE) * (H / TILE) >= 256 ? 4
+                 : ppo::ceil_div(Bm, 2 * TILE) * (H / TILE) >= 256 ? 2 : 1;
+  const dim3 grid(ppo::ceil_div(Bm, rt * TILE), H / TILE);
+#define PPO_GRU_STEP_X(NIT)                                                                                    \
+  if (rt == 4) hipLaunchKernelGGL((gru_step_x_kernel<NIT, 4>), grid, dim3(256), 0, st, a);                     \
+  else if (rt == 2) hipLaunchKernelGGL((gru_step_x_kernel<NIT, 2>), grid, dim3(256), 0, st, a);                \
+  else hipLaunchKernelGGL((gru_step_x_kernel<NIT, 1>), grid, dim3(256), 0, st, a);
   switch (I == H ? H / 64 : 0) {  // 16-wide k steps per wave of both contractions
-    case 1: hipLaunchKernelGGL((gru_fwd_step_kernel<1, true>), grid, dim3(256), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((gru_fwd_step_kernel<2, true>), grid, dim3(256), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((gru_fwd_step_kernel<4, true>), grid, dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL((gru_fwd_step_kernel<0, true>), grid, dim3(256), 0, st, a); break;
+    case 1: PPO_GRU_STEP_X(1) break;
+    case 2: PPO_GRU_STEP_X(2) break;
+    case 4: PPO_GRU_STEP_X(4) break;
+    default: PPO_GRU_STEP_X(0) break;
   }
+#undef PPO_GRU_STEP_X
   return ppo::check_launch("ppo_gru_fwd_step_x_f32");
 }
 

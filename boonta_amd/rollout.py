@@ -231,7 +231,7 @@ class RecurrentStepExecutor(ForwardChain):
     launches, one for the GRU step with its input projections (a trunk width that
     is a multiple of 64), one for the head and the draw (at most 15 logits);
     ``fused=False`` issues the projection GEMM, the head GEMM and the sampling
-    launch instead (128 -> 256 -> GRU 256, 1024 envs: 43 -> 31
+    launch instead (128 -> 256 -> GRU 256, 1024 envs: 42 -> 28
     us a step, a key copy left out besides)."""
 
     def __init__(self, program: Program, flat: FlatState, rows: int, fused: bool | None = None):
