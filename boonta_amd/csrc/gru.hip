@@ -1164,9 +1164,11 @@ PPO_EXPORT int ppo_gru_fwd_step_x_f32(void* stream, const float* x, int64_t ldx,
     return ppo::set_error(PPO_ERR_ARG, "ppo_gru_fwd_step_x_f32: x and hprev rows must be 16-byte aligned");
   XStepArgs a{x, ldx, I, wi, ldwi, bi, hprev, ldh, terminated, truncated, wh, ldwh, bhn, h_out, ldo, Bm, H};
   hipStream_t st = ppo::as_stream(stream);
-  // the most row tiles per workgroup that leave one workgroup per CU
-  const int rt = ppo::ceil_div(Bm, 4 * TILE) * (H / TILE) >= 256 ? 4
-                 : ppo::ceil_div(Bm, 2 * TILE) * (H / TILE) >= 256 ? 2 : 1;
+  // the most row tiles per workgroup that leave two workgroups per CU (1024
+  // sequences of 256 units: two tiles 27.7 us a step called from the host, four, one
+  // workgroup per CU, 28.2; replayed alone the launch takes 17.0 and 16.5)
+  const int rt = ppo::ceil_div(Bm, 4 * TILE) * (H / TILE) >= 512 ? 4
+                 : ppo::ceil_div(Bm, 2 * TILE) * (H / TILE) >= 512 ? 2 : 1;
   const dim3 grid(ppo::ceil_div(Bm, rt * TILE), H / TILE);
 #define PPO_GRU_STEP_X(NIT)                                                                                    \
   if (rt == 4) hipLaunchKernelGGL((gru_step_x_kernel<NIT, 4>), grid, dim3(256), 0, st, a);                     \

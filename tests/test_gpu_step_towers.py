@@ -121,8 +121,8 @@ def test_shared_head_and_draw_in_one_launch(rows, width, depth, A, temperature):
 
 
 @pytest.mark.parametrize("rows,H,I,A", [(1, 64, 64, 2), (17, 128, 128, 15), (33, 256, 256, 8), (300, 256, 64, 3),
-                                        (16, 512, 512, 4), (40, 64, 192, 5), (40, 64, 96, 16), (500, 256, 256, 3),
-                                        (1000, 256, 256, 4), (2000, 128, 128, 5), (460, 512, 64, 2)])
+                                        (16, 512, 512, 4), (40, 64, 192, 5), (40, 64, 96, 16), (1000, 256, 256, 3),
+                                        (2040, 256, 256, 4), (4090, 128, 128, 5), (500, 512, 64, 2)])
 def test_recurrent_step_forms_the_projections(rows, H, I, A):
     """ppo_gru_fwd_step_x_f32 against the oracle and the projection GEMM's path,
     with rows reset, at equal and unequal widths (96: not its multiple of 64) and
