@@ -463,12 +463,6 @@ class ForwardChain:
     CHAIN16 = True
     CHAIN16_BWD = True
     DW16_SIDE = True  # the chain group's later weight gradients beside the first layer's, on the side stream
-    DW_SIDE = True    # fp32: a later layer's weight gradient beside its input cotangent, on the side stream
-    # ... from this many multiply-adds on (65536 rows of 512 x 512: 5066 us an update of 4 steps against 5083 on one
-    # stream).  Below it the fork and join cost more than the overlap gives: the two contractions fill the chip each
-    # (32768 rows of 256 x 256 the same either way), or are a few us long (2 x 256 tanh trunk, 4 steps of 128 rows: 378
-    # us against 321; of 4096, 450 against 416; of 8192, 523 against 488).
-    DW_SIDE_WORK = 65536 * 512 * 512
     # every weight gradient of the chain group in one launch (ppo_gemm_bf16s_dw_group):
     # the later layers' few tiles run beside the first layer's 198, with no
     # stream fork and join around them
@@ -1299,10 +1293,12 @@ class MLPExecutor(ForwardChain):
         g["args"] = [ctypes.addressof(g[k]) for k in order]
         return g
 
-    def _bwd_layers(self, st, layers, x0, ldx0, idx0, side_dw=False):
+    def _bwd_layers(self, st, layers, x0, ldx0, idx0):
         """Back-propagates through layers whose last output cotangent is in
-        place; with side_dw (st the main stream) the fp32 weight gradient of a
-        large later layer runs on the side stream beside its input cotangent."""
+        place, on one stream: a later layer's weight gradient beside its input
+        cotangent gained 0.3 % at 65536 x 512 x 512 multiply-adds and cost 5-18
+        % at small minibatches, and a replay of such a graph (three layers, two
+        branches a step) ended in a host fault whose cause is not known."""
         c = layers[0].chain16 if layers else None
         if c is not None and c["bwd"]:
             # every LayerNorm backward and input cotangent in one launch; then
@@ -1347,7 +1343,6 @@ class MLPExecutor(ForwardChain):
                 x, ldx, ridx = x0, ldx0, idx0
             obs16 = i == 0 and self._reads_obs16(x, ridx, 0)
             y16 = i > 0 and layers[i - 1].Y16 is not None
-            sd = st
             # bf16 cotangent of a LayerNorm layer: read by its dW and dX contractions
             dz16 = s.ln is not None and lb.dZ16 is not None and (obs16 or i > 0)
             if s.ln is not None:
@@ -1368,11 +1363,7 @@ class MLPExecutor(ForwardChain):
             elif i == 0 and self._first_dw_final(st, layers, x, ldx, ridx):
                 pass   # the first layer's weight gradient with every leaf's gradient assembly
             else:
-                # a large later layer's weight gradient runs on the side stream
-                # beside its input cotangent (neither writes what the other reads)
-                if i > 0 and side_dw and self.DW_SIDE and self.mb * d.fin * s.ld >= self.DW_SIDE_WORK:
-                    sd = self._fork(st)
-                self._gemm(sd, A_COL, B_KN, x, ldx, ridx, _p(lb.dZ), s.ld, _p(lb.wpart), s.ld, d.fin,
+                self._gemm(st, A_COL, B_KN, x, ldx, ridx, _p(lb.dZ), s.ld, _p(lb.wpart), s.ld, d.fin,
                           s.ld, self.mb, lb.splits, d.fin * s.ld, EPI_STORE, None, 0, None, None, 0, _p(lb.bpart),
                           -1)
             if i > 0:
@@ -1385,8 +1376,6 @@ class MLPExecutor(ForwardChain):
                     self._gemm(st, A_ROW, B_NK, _p(lb.dZ), s.ld, None, self.flat.view(d.w), d.w.ld,
                               dst, layers[i - 1].spec.ld, self.mb, d.fin, s.ld, 1, 0, epi, None, act, None, aux,
                               ldaux, None, -1)
-            if sd != st:
-                self._join(st, sd)
 
     def _fwd_boot_chain(self, st, x, ldx, nrows):
         """The critic tower's forward for the bootstrap rows in one launch."""
@@ -1791,7 +1780,7 @@ class MLPExecutor(ForwardChain):
             if prog.shared_head:
                 self._fwd_layers(st, self.trunk, obs, ldo, idx, mb)
                 self._fused_head_loss(st, idx, step, dist, A, scale_ptr, act_i, act_f)
-                self._bwd_layers(st, self.trunk, obs, ldo, idx, side_dw=True)
+                self._bwd_layers(st, self.trunk, obs, ldo, idx)
             elif self.chain_act:
                 t, s0, pre = self._act, self.actor[0].spec, self._head_loss_args
                 # (the zero-padded copy's rows take 16-byte loads)
@@ -1844,7 +1833,7 @@ class MLPExecutor(ForwardChain):
                       int(cfg.clip_value_loss), float(cfg.entropy_coefficient), float(cfg.value_coefficient), 1.0)
             self._head_back(st, self.trunk, self.DHEAD, h, self.HWPART, self.HBPART, self.head_splits, hx, ldhx,
                             hidx)
-            self._bwd_layers(st, self.trunk, obs, ldo, idx, side_dw=True)
+            self._bwd_layers(st, self.trunk, obs, ldo, idx)
         else:
             ha, hc = prog.head_a, prog.head_c
             s2 = self._fork(st)

@@ -102,6 +102,29 @@ def test_recorded_launches_match_the_c_signatures(config):
             assert all((ha, wa, ba, dha, wpa, bpa, stats))
 
 
+def test_a_shared_trunk_update_stays_on_one_stream():
+    """A float32 shared trunk of three layers issues every launch of an update
+    on the caller's stream (no branch beside the input cotangents, whatever
+    the size)."""
+    from types import SimpleNamespace
+    from boonta_amd import networks as nn
+    r = small(2)
+    layers = [f(x) for _ in range(3) for f, x in ((nn.Dense, 64), (lambda _: nn.tanh, 0))]
+    net = nn.Network(feature_extractor=nn.FeatureExtractor(nn.Sequential(layers)),
+                     head=nn.ActorCritic(actor=nn.Categorical(nn.Dense(6)), critic=nn.Dense(1)))
+    prog = Program(net.plan(r.obs_dim))
+    ex = executor(r, prog, FlatState(prog, torch.device("cpu")))
+    ex.side, ex._ev_fork, ex._ev_join = SimpleNamespace(cuda_stream=99), 1, 2
+    ex.DW_SIDE_WORK = 0
+    ex.bind(fake_inputs(ex))
+    calls = []
+    ex._call = lambda name, *args: calls.append((name, args))
+    ex.issue(7)
+    assert [n for n, _ in calls].count("ppo_gemm_f32") > 6
+    assert not [n for n, _ in calls if n == "ppo_stream_wait"]
+    assert {args[0] for _, args in calls} == {7}
+
+
 @pytest.mark.parametrize("config", ALL_CONFIGS)
 def test_flat_layout_round_trips_the_parameter_tree(config):
     r = recipes.make(config)
