@@ -17,18 +17,20 @@
 // lane half h holds k = 8g + 4h + s (both operands the same order, so the sum
 // is unchanged).
 //
-// Products: v_mfma_f32_32x32x2_f32 for small row-layout problems; else each
-// wave splits the fp32 values it reads from LDS into three bf16 pieces and
-// multiplies those (split_f32.h): six v_mfma_f32_32x32x16_bf16 replace eight
-// fp32 ones at 3/8 of their cycles, and 11 vector instructions per pair of
-// operand values beside them.  With 64 x 64 outputs per wave the matrix cores
-// and the vector unit are about evenly busy (228 TFLOP/s of fp32 products in
-// registers, 151 on fp32 MFMA, 285 without the splitting).  32768 x 256 x 256
-// forward on 256 x 128 tiles 42.6 -> 32-34 us, x 400 with gathered rows 65.7 ->
-// 47, input cotangent 57 -> 41 (tile 2), 256 x 256 x 32768 weight gradient on
-// 64 splits 46 -> 38, 400 x 256 x 32768 on 64 x 64 tiles 83 -> 68.  What is left
-// is the stage barriers and the epilogue of a grid that runs one wave of
-// workgroups.
+// Products: v_mfma_f32_32x32x2_f32; in the row layouts' wide tiles (2, 8, 9)
+// each wave splits the fp32 values it reads from LDS into three bf16 pieces and
+// multiplies those (split_f32.h): eight v_mfma_f32_32x32x16_bf16 replace eight
+// fp32 ones at half their cycles, and 13 vector instructions per pair of
+// operand values beside them.  The leading products keep an accumulator of
+// their own, so an output rounds once per 16 reduction elements at its own
+// size, the other seven at 2^-8 of it: errors against float64 of 0.3-0.4 times
+// those of fp32 MFMA (normal operands, K = 400: 1.9 x 2^-24 against 6.0).
+// 32768 x 256 x 256 forward on 256 x 128 tiles 42.2 us on fp32 MFMA, 38.4
+// split, x 400 63.4 and 56.4, input cotangent 46.2 (64 x 64 tiles) and 41.2
+// (tile 2).  (Six products: 31.6, 46.5 and 35.0, with up to half a last place
+// of a product lost.)  What is left is the splitting, which runs before the
+// MFMAs rather than beside them, the stage barriers and the epilogue of a grid
+// of one wave of workgroups.
 // LDS layouts (fp32, 16-byte chunks XOR-swizzled on the copy side):
 //   k-contiguous [ROWS][32]: chunk c of row r at c ^ kc_swizzle(r); an operand
 //     read (4 consecutive k of one row) is one 16-byte read;
@@ -154,7 +156,7 @@ __device__ __forceinline__ floatx4 operand(const float* lds, int rbase, int g, i
 // A wave's MB x NB blocks from row wm0 and column wn0 over reduction [kb, ke)
 // on v_mfma_f32_32x32x2_f32, operands straight from global memory: the cold
 // path of sums that the split products left not finite.
-template <int MB, int NB, bool A_K, bool B_K>
+template <int MB, int NB, bool B_K>
 __device__ __forceinline__ void exact_wave_tile(const GemmParams& p, floatx16 (&acc)[MB][NB], int wm0, int wn0, int kb,
                                                 int ke, int lane) {
   const int h = lane >> 5, l32 = lane & 31;
@@ -173,9 +175,8 @@ __device__ __forceinline__ void exact_wave_tile(const GemmParams& p, floatx16 (&
 #pragma unroll
     for (int bi = 0; bi < MB; ++bi) {
       const int m = min(wm0 + bi * 32 + l32, p.M - 1);
-      const int64_t r = A_K ? m : kc;
-      const int64_t row = p.rows ? (int64_t)p.rows[r] : r;
-      a[bi] = in ? p.A[row * p.lda + (A_K ? kc : m)] : 0.f;
+      const int64_t row = p.rows ? p.rows[m] : m;
+      a[bi] = in ? p.A[row * p.lda + kc] : 0.f;
     }
 #pragma unroll
     for (int bj = 0; bj < NB; ++bj) {
@@ -202,6 +203,7 @@ template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, int NBUF, bool SPL
 __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int tn, int split) {
   constexpr int NW = WM * WN;
   constexpr int MB = BM / WM / 32, NB = BN / WN / 32;  // 32 x 32 blocks per wave
+  static_assert(!SPLIT || A_K, "row layouts only: the cold path's reads, no bias gradient");
   static_assert(MB * WM * 32 == BM && NB * WN * 32 == BN, "tile must split into 32 x 32 blocks");
   using OpA = Operand<BM, A_K, NW>;
   using OpB = Operand<BN, B_K, NW>;
@@ -225,6 +227,16 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  // SPLIT: the sums of every piece product but the leading ones
+  floatx16 low[SPLIT ? MB : 1][SPLIT ? NB : 1];
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) low[i][j][r] = 0.f;
+  }
   float bsum[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j) bsum[j] = 0.f;
@@ -328,43 +340,39 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
         }
       }
     } else {
-      // a 16-deep block of the reduction (two groups per lane half), the next
-      // block's LDS reads issued before this block's products
-      floatx4 a4[2][2][MB], b4[2][2][NB];
-      auto read_ops = [&](int set, int blk) {
+      // a 16-deep block of the reduction (two groups per lane half); the next
+      // block's LDS reads are issued once this block's operands are split,
+      // ahead of its products
+      floatx4 a4[2][MB], b4[2][NB];
+      auto read_ops = [&](int blk) {
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
 #pragma unroll
           for (int bi = 0; bi < MB; ++bi)
-            a4[set][q][bi] = operand<BM, A_K>(la, wm * (BM / WM) + bi * 32, 2 * blk + q, lane);
+            a4[q][bi] = operand<BM, A_K>(la, wm * (BM / WM) + bi * 32, 2 * blk + q, lane);
 #pragma unroll
           for (int bj = 0; bj < NB; ++bj)
-            b4[set][q][bj] = operand<BN, B_K>(lb, wn * (BN / WN) + bj * 32, 2 * blk + q, lane);
+            b4[q][bj] = operand<BN, B_K>(lb, wn * (BN / WN) + bj * 32, 2 * blk + q, lane);
         }
       };
-      read_ops(0, 0);
+      read_ops(0);
 #pragma unroll
       for (int blk = 0; blk < BK / 16; ++blk) {
-        const int cur = blk & 1;
-        if (blk + 1 < BK / 16) read_ops(cur ^ 1, blk + 1);
         ppo::Split8 fa[MB], fb[NB];
 #pragma unroll
-        for (int bi = 0; bi < MB; ++bi) fa[bi] = ppo::split8(a4[cur][0][bi], a4[cur][1][bi]);
+        for (int bi = 0; bi < MB; ++bi) fa[bi] = ppo::split8(a4[0][bi], a4[1][bi]);
 #pragma unroll
-        for (int bj = 0; bj < NB; ++bj) fb[bj] = ppo::split8(b4[cur][0][bj], b4[cur][1][bj]);
+        for (int bj = 0; bj < NB; ++bj) fb[bj] = ppo::split8(b4[0][bj], b4[1][bj]);
+        if (blk + 1 < BK / 16) read_ops(blk + 1);
 #pragma unroll
         for (int t = 0; t < ppo::SPLIT_PRODUCTS; ++t)
 #pragma unroll
           for (int bi = 0; bi < MB; ++bi)
 #pragma unroll
-            for (int bj = 0; bj < NB; ++bj) acc[bi][bj] = ppo::split_mfma(t, fa[bi], fb[bj], acc[bi][bj]);
-        if (do_bsum) {
-#pragma unroll
-          for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int bj = 0; bj < NB; ++bj)
-              bsum[bj] += (b4[cur][q][bj][0] + b4[cur][q][bj][1]) + (b4[cur][q][bj][2] + b4[cur][q][bj][3]);
-        }
+            for (int bj = 0; bj < NB; ++bj) {
+              floatx16& c = t + 1 < ppo::SPLIT_PRODUCTS ? low[bi][bj] : acc[bi][bj];
+              c = ppo::split_mfma(t, fa[bi], fb[bj], c);
+            }
       }
     }
   }
@@ -378,9 +386,20 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
 #pragma unroll
       for (int bj = 0; bj < NB; ++bj)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) nonfinite = __fmaf_rn(acc[bi][bj][r], 0.f, nonfinite);
-    if (__builtin_expect(__any(nonfinite != 0.f), 0))
-      exact_wave_tile<MB, NB, A_K, B_K>(p, acc, m0 + wm * (BM / WM), n0 + wn * (BN / WN), kb, ke, lane);
+        for (int r = 0; r < 16; ++r) {
+          acc[bi][bj][r] += low[bi][bj][r];
+          nonfinite = __fmaf_rn(acc[bi][bj][r], 0.f, nonfinite);
+        }
+    if (__builtin_expect(__any(nonfinite != 0.f), 0)) {
+      exact_wave_tile<MB, NB, B_K>(p, acc, m0 + wm * (BM / WM), n0 + wn * (BN / WN), kb, ke, lane);
+    } else {
+#pragma unroll
+      for (int bi = 0; bi < MB; ++bi)
+#pragma unroll
+        for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[bi][bj][r] *= ppo::SPLIT_UNSCALE;
+    }
   }
 
   if constexpr (WT)
@@ -414,8 +433,8 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32d_group_kernel(F32Group 
   int i = 0;
   while (i + 1 < g.count && t >= g.start[i + 1]) ++i;
   const int local = t - g.start[i];
-  gemm_f32d_tile<BM, BN, WM, WN, A_K, B_K, NBUF, true>(g.p[i], (local / g.gx[i]) % g.gy[i], local % g.gx[i],
-                                                 local / (g.gx[i] * g.gy[i]));
+  gemm_f32d_tile<BM, BN, WM, WN, A_K, B_K, NBUF, false>(g.p[i], (local / g.gx[i]) % g.gy[i], local % g.gx[i],
+                                                  local / (g.gx[i] * g.gy[i]));
 }
 
 // The split-K counts the finishing sum is compiled for.
@@ -448,7 +467,7 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32d_group_final_kernel(F32
   const GemmParams& p = g.p[i];
   const int local = t - g.start[i];
   const int tm = (local / g.gx[i]) % g.gy[i], tn = local % g.gx[i];
-  gemm_f32d_tile<BM, BN, WM, WN, false, false, NBUF, true, KIDX, true>(p, tm, tn, local / (g.gx[i] * g.gy[i]));
+  gemm_f32d_tile<BM, BN, WM, WN, false, false, NBUF, false, KIDX, true>(p, tm, tn, local / (g.gx[i] * g.gy[i]));
   // every wave's partial stores complete, then one arrival for the tile
   const int slot = f.slot0[i] + tm * g.gx[i] + tn;
   double sq = 0.0;
@@ -484,7 +503,7 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32d_group_final_kernel(F32
   ppo_gr::block_sumsq<WM * WN * 64>(sq, s_w, f.sumsq + slot);
 }
 
-template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, bool SPLIT = true>
+template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, bool SPLIT = false>
 int launch(hipStream_t st, const GemmParams& p, int splits) {
   constexpr int NBUF = WM * WN == 4 ? 2 : 3;
   dim3 grid(ppo::ceil_div(p.N, BN), ppo::ceil_div(p.M, BM), splits * p.towers);
@@ -492,34 +511,20 @@ int launch(hipStream_t st, const GemmParams& p, int splits) {
   return ppo::check_launch("ppo_gemm_f32");
 }
 
-// Whether a problem's products run on the bf16 matrix cores.  Weight
-// gradients always; the row layouts from 2^21 outputs on: there the matrix
-// cores bound the launch (32768 x 256 x 256 forward on 64 x 64 tiles 45.7 ->
-// 39.4 us, 4096 x 512 x 512 27.5 -> 24.6), below it latency does and the
-// splitting's vector work is in the way (2048 x 256 x 256 x two towers 13.2
-// -> 13.6 us, 1024 x 768 x 256 10.1 -> 10.1).  By the problem's size
-// alone, so every tile of one problem forms the same bits (tiles 1, 2, 8 and
-// 9, which only large problems take, are compiled split).
-template <bool A_K>
-bool split_products(const GemmParams& p) {
-  return !A_K || (int64_t)p.M * p.N >= (1 << 21);
-}
-
+// The row layouts' wide tiles form their products on the bf16 matrix cores;
+// the narrow ones, whose waves split each operand value for 32 or 64 outputs
+// only, and the weight gradients lose by it what they gain (64 x 64 tiles:
+// 16384 x 256 x 400 forward 38.2 us on fp32 MFMA, 39.4 split; 256 x 256 weight
+// gradient of 2048 rows 7.2 and 7.9).
 template <bool A_K, bool B_K>
 int launch_tile(hipStream_t st, const GemmParams& p, int splits, int tile) {
   switch (tile) {
-    case 0:
-      if constexpr (A_K)
-        if (!split_products<A_K>(p)) return launch<128, 128, 2, 2, A_K, B_K, false>(st, p, splits);
-      return launch<128, 128, 2, 2, A_K, B_K>(st, p, splits);
+    case 0: return launch<128, 128, 2, 2, A_K, B_K>(st, p, splits);
     case 1: return launch<128, 64, 2, 2, A_K, B_K>(st, p, splits);
-    case 2: return launch<64, 128, 2, 2, A_K, B_K>(st, p, splits);
-    case 8: return launch<128, 256, 2, 4, A_K, B_K>(st, p, splits);
-    case 9: return launch<256, 128, 4, 2, A_K, B_K>(st, p, splits);
-    default:
-      if constexpr (A_K)
-        if (!split_products<A_K>(p)) return launch<64, 64, 2, 2, A_K, B_K, false>(st, p, splits);
-      return launch<64, 64, 2, 2, A_K, B_K>(st, p, splits);
+    case 2: return launch<64, 128, 2, 2, A_K, B_K, A_K>(st, p, splits);
+    case 8: return launch<128, 256, 2, 4, A_K, B_K, A_K>(st, p, splits);
+    case 9: return launch<256, 128, 4, 2, A_K, B_K, A_K>(st, p, splits);
+    default: return launch<64, 64, 2, 2, A_K, B_K>(st, p, splits);
   }
 }
 
