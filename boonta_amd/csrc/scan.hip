@@ -28,7 +28,11 @@
 // each composes the maps before it (in time order for the forward, in reverse
 // for the backward) to write its chunk's outputs from the exact carry.
 // Sequences of up to 128 steps are one such tile of 16 chunks, longer ones run
-// tile after tile.
+// tile after tile.  A chunk's decay is the product of its steps' and can leave
+// float32's range where no state does: a tile of a long sequence whose composed
+// state is not finite is stepped through instead; one tile alone (9 to 128
+// steps) is not.  Below the range the product rounds to the subnormals' grid, at
+// most 2^-149 of the state entering the chunk.
 #include "split_f32.h"
 
 #include <algorithm>
@@ -347,6 +351,45 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // Bit i: step t0 + i (below steps) of sequence n restarts.
 __device__ __forceinline__ uint32_t done_bits(uint8_t flag, bool live) { return (uint32_t)__ballot(live && flag); }
 
+// Whether a lane's state after a tile is not finite.  Every wave composes the
+// same maps, so all take the same way.
+template <int VW>
+__device__ __forceinline__ bool any_nonfinite(const float (&x)[VW]) {
+  float z = 0.f;
+#pragma unroll
+  for (int k = 0; k < VW; ++k) z = __fmaf_rn(x[k], 0.f, z);
+  return __any(z != 0.f);
+}
+
+// The states entering (mine) and leaving (x) a tile from the one entering it
+// (x), chunk after chunk, each by its own wave a step at a time: the cold path
+// of a tile whose composed state is not finite.  A map's decay can overflow (or
+// its sum) where no step does: eight decays of 1e5 from a zero state are
+// inf * 0.  pa, pb: LDS that every wave has read past.
+template <int C, int TL, int VW, bool REVERSE>
+__device__ __forceinline__ void step_by_step(const float (&a)[TL][VW], const float (&b)[TL][VW], float (&x)[VW],
+                                             float (&mine)[VW], float* pa, float* pb, int c, int lane) {
+  lds_barrier();
+#pragma unroll 1
+  for (int i = 0; i < C; ++i) {
+    float* slot = (i & 1 ? pb : pa) + lane * VW;
+    if (c == (REVERSE ? C - 1 - i : i)) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) mine[k] = x[k];
+#pragma unroll
+      for (int j = 0; j < TL; ++j)
+#pragma unroll
+        for (int k = 0; k < VW; ++k)
+          x[k] = a[REVERSE ? TL - 1 - j : j][k] * x[k] + b[REVERSE ? TL - 1 - j : j][k];
+#pragma unroll
+      for (int k = 0; k < VW; ++k) slot[k] = x[k];
+    }
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < VW; ++k) x[k] = slot[k];
+  }
+}
+
 template <typename S, int VW>
 __global__ void __launch_bounds__(64 * TILE_WAVES) scan_fwd_tile_kernel(ScanArgs p) {
   __shared__ float sA[2][TILE_WAVES * 64 * VW], sB[2][TILE_WAVES * 64 * VW];
@@ -421,7 +464,9 @@ __global__ void __launch_bounds__(64 * TILE_WAVES) scan_fwd_tile_kernel(ScanArgs
     }
     if (t0 - c * TL + tile < p.steps) fetch(set ^ 1, t0 + tile);
     lds_barrier();
-    float hc[VW];
+    float hc[VW], hs[VW];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) hs[k] = h[k];
 #pragma unroll
     for (int cc = 0; cc < C; ++cc) {
       if (cc == c) {
@@ -430,6 +475,11 @@ __global__ void __launch_bounds__(64 * TILE_WAVES) scan_fwd_tile_kernel(ScanArgs
       }
 #pragma unroll
       for (int k = 0; k < VW; ++k) h[k] = pa[(cc * 64 + lane) * VW + k] * h[k] + pb[(cc * 64 + lane) * VW + k];
+    }
+    if (__builtin_expect(any_nonfinite(h), 0)) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) h[k] = hs[k];
+      step_by_step<C, TL, VW, false>(av, bv, h, hc, pa, pb, c, lane);
     }
 #pragma unroll
     for (int i = 0; i < TL; ++i) {
@@ -513,7 +563,9 @@ __global__ void __launch_bounds__(64 * TILE_WAVES) scan_bwd_tile_kernel(ScanArgs
     }
     if (it > 0) fetch(set ^ 1, t0 - tile);
     lds_barrier();
-    float dc[VW];
+    float dc[VW], ds[VW];
+#pragma unroll
+    for (int k = 0; k < VW; ++k) ds[k] = d[k];
 #pragma unroll
     for (int cc = C - 1; cc >= 0; --cc) {
       if (cc == c) {
@@ -522,6 +574,11 @@ __global__ void __launch_bounds__(64 * TILE_WAVES) scan_bwd_tile_kernel(ScanArgs
       }
 #pragma unroll
       for (int k = 0; k < VW; ++k) d[k] = pa[(cc * 64 + lane) * VW + k] * d[k] + pb[(cc * 64 + lane) * VW + k];
+    }
+    if (__builtin_expect(any_nonfinite(d), 0)) {
+#pragma unroll
+      for (int k = 0; k < VW; ++k) d[k] = ds[k];
+      step_by_step<C, TL, VW, true>(al, gv, d, dc, pa, pb, c, lane);
     }
 #pragma unroll
     for (int i = TL - 1; i >= 0; --i) {

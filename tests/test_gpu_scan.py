@@ -219,3 +219,44 @@ def test_long_sequences_run_tile_after_tile(batch, steps, features, dtype, offse
     for got, exp in zip((h, *grads), (want, da, db, db[:, 0] * A[:, 0])):
         got = got.detach().double().cpu()
         assert float((got - exp).norm()) <= rel * float(exp.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("steps, features", [(200, 64), (333, 7), (1000, 100)])
+@pytest.mark.parametrize("resets", [False, True])
+def test_decays_whose_product_overflows_leave_finite_states_finite(dtype, steps, features, resets):
+    """Long sequences whose chunks' decays multiply past float32's range while no
+    state or cotangent does: a zero state through forty decays of 1e5, and one of
+    1e-15 raised by 1e40 and brought back."""
+    g = torch.Generator().manual_seed(steps)
+    batch = 3
+    a = torch.rand(batch, steps, features, generator=g) * 0.9 + 0.05
+    b = torch.randn(batch, steps, features, generator=g)
+    a[:, 20:60], b[:, :60] = 1e5, 0.0
+    a[:, 90], a[:, 98:100], a[:, 100:102], b[:, 90:106] = 1e-15, 1e20, 1e-20, 0.0
+    cot = torch.randn(batch, steps, features, generator=g)
+    cot[:, 20:] = 0.0
+    done = torch.zeros(batch, steps, dtype=torch.bool)
+    done[:, steps - 20] = resets
+    a, b, init, cot = (x.to(dtype).cuda() for x in (a, b, torch.zeros(batch, features), cot))
+    for x in (a, b, init):
+        x.requires_grad_(True)
+    h = ssm_scan(a, b, done.cuda(), init) if resets else scan(a, b, init)
+    grads = torch.autograd.grad(h, (a, b, init), cot)
+    A, B, W = (x.detach().double().cpu() for x in (a, b, cot))
+    A = torch.where(done[:, :, None], 0.0, A)
+    want, s = torch.empty_like(A), torch.zeros(batch, features, dtype=torch.float64)
+    for t in range(steps):
+        s = A[:, t] * s + B[:, t]
+        want[:, t] = s
+    db, d = torch.empty_like(A), torch.zeros_like(s)
+    for t in range(steps - 1, -1, -1):
+        d = W[:, t] + (A[:, t + 1] * d if t + 1 < steps else 0.0)
+        db[:, t] = d
+    da = db * torch.cat([torch.zeros(batch, 1, features, dtype=torch.float64), want[:, :-1]], 1)
+    rel = 4e-6 if dtype == torch.float32 else 1e-2
+    for got, exp in zip((h, *grads), (want, da, db, db[:, 0] * A[:, 0])):
+        got = got.detach().double().cpu()
+        assert bool(torch.isfinite(got).all())
+        axes = (0, 2) if got.ndim == 3 else None  # a step's own norm: the states span forty decades
+        assert bool(((got - exp).norm(dim=axes) <= rel * exp.norm(dim=axes)).all())
