@@ -1169,17 +1169,29 @@ PPO_EXPORT int ppo_gru_fwd_step_x_f32(void* stream, const float* x, int64_t ldx,
   // workgroup per CU, 28.2; replayed alone the launch takes 17.0 and 16.5)
   const int rt = ppo::ceil_div(Bm, 4 * TILE) * (H / TILE) >= 512 ? 4
                  : ppo::ceil_div(Bm, 2 * TILE) * (H / TILE) >= 512 ? 2 : 1;
+  // 16-wide k steps per wave of both contractions, all loaded ahead of the
+  // first product; not four of them for four row tiles, whose operands (320
+  // registers) leave one workgroup per CU (256 -> 256, whole steps of 4096 and
+  // 16384 sequences: 71 and 260 us with them, 59 and 198 with a loop; the
+  // projection GEMM and the step apart 71 and 195)
+  const int nit = I == H && (H / 64 < 4 || rt < 4) ? H / 64 : 0;
   const dim3 grid(ppo::ceil_div(Bm, rt * TILE), H / TILE);
-#define PPO_GRU_STEP_X(NIT)                                                                                    \
-  if (rt == 4) hipLaunchKernelGGL((gru_step_x_kernel<NIT, 4>), grid, dim3(256), 0, st, a);                     \
-  else if (rt == 2) hipLaunchKernelGGL((gru_step_x_kernel<NIT, 2>), grid, dim3(256), 0, st, a);                \
-  else hipLaunchKernelGGL((gru_step_x_kernel<NIT, 1>), grid, dim3(256), 0, st, a);
-  switch (I == H ? H / 64 : 0) {  // 16-wide k steps per wave of both contractions
-    case 1: PPO_GRU_STEP_X(1) break;
-    case 2: PPO_GRU_STEP_X(2) break;
-    case 4: PPO_GRU_STEP_X(4) break;
-    default: PPO_GRU_STEP_X(0) break;
+#define PPO_GRU_STEP_X(NIT, RT) \
+  hipLaunchKernelGGL((gru_step_x_kernel<NIT, RT>), grid, dim3(256), 0, st, a);
+#define PPO_GRU_STEP_X_RT(NIT)                \
+  if (rt == 4) { PPO_GRU_STEP_X(NIT, 4) }      \
+  else if (rt == 2) { PPO_GRU_STEP_X(NIT, 2) } \
+  else { PPO_GRU_STEP_X(NIT, 1) }
+  switch (nit) {
+    case 1: PPO_GRU_STEP_X_RT(1) break;
+    case 2: PPO_GRU_STEP_X_RT(2) break;
+    case 4:
+      if (rt == 2) { PPO_GRU_STEP_X(4, 2) }
+      else { PPO_GRU_STEP_X(4, 1) }
+      break;
+    default: PPO_GRU_STEP_X_RT(0) break;
   }
+#undef PPO_GRU_STEP_X_RT
 #undef PPO_GRU_STEP_X
   return ppo::check_launch("ppo_gru_fwd_step_x_f32");
 }
