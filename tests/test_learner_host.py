@@ -147,6 +147,37 @@ def test_flat_layout_round_trips_the_parameter_tree(config):
     assert prog.layout.size % 64 == 0
 
 
+class ActChainExecutor(MLPExecutor):
+    CHAIN_ACT = True  # (on host memory too)
+
+
+def tower_program(width, depth, obs):
+    from boonta_amd import networks as nn
+    torso = lambda: [f for _ in range(depth) for f in (nn.Dense(width), nn.tanh)]
+    net = nn.Network(feature_extractor=nn.FeatureExtractor(nn.Identity()),
+                     head=nn.ActorCritic(actor=nn.Categorical(nn.Sequential(torso() + [nn.Dense(6)])),
+                                         critic=nn.Sequential(torso() + [nn.Dense(1)])))
+    return Program(net.plan(obs))
+
+
+@pytest.mark.parametrize("width, depth, obs, rows", [(64, 1, 20, 4096), (64, 3, 376, 8192), (128, 1, 87, 2048),
+                                                     (128, 3, 376, 4096), (256, 1, 20, 2048), (256, 2, 87, 4096),
+                                                     (256, 3, 376, 2048)])
+def test_plain_towers_leave_their_one_launch_update_past_its_rounds(width, depth, obs, rows):
+    """The largest minibatch of the launch, and one row tile more layer by layer."""
+    from dataclasses import replace
+    r = recipes.make(1)
+    cfg = replace(r.cfg, num_minibatches=1, update_epochs=1)
+    prog = tower_program(width, depth, obs)
+    flat = FlatState(prog, torch.device("cpu"))
+    for n, chain in ((rows, True), (rows + 16, False)):
+        ex = ActChainExecutor(prog, flat, cfg, r.optimizer, 1, n)
+        ex.bind(fake_inputs(ex))
+        names = [c for c, _ in ex.record()]
+        assert names.count("ppo_mlp_act_fwd_head_loss_bwd_f32") == int(chain)
+        assert names.count("ppo_head_loss_f32") == int(not chain)
+
+
 def test_shared_heads_pack_logits_and_value_in_one_matrix():
     r = recipes.make(2)
     prog = Program(r.network.plan(r.obs_dim))
