@@ -104,9 +104,12 @@ class StepExecutor(ForwardChain):
         return {"keep": keep, "args": (n, *map(ctypes.addressof, keep), _act(prog.trunk[0].act), view(h.w), h.w.ld)}
 
     def _towers_fusable(self, lib) -> bool:
-        """Whether the paired towers' one-launch step covers this program: for
-        every number of rows it replaces two launches per layer and three after
-        (4 x 256 LayerNorm + SiLU, 4096 rows: 125 -> 64 us)."""
+        """Whether the paired towers' one-launch step covers this program: it
+        replaces two launches per layer and three after (4 x 256 LayerNorm +
+        SiLU, 4096 rows: 125 -> 64 us, 65536: 1144 -> 937; 2 x 64 and 2 x 128
+        tanh, 65536: 150 -> 67 and 207 -> 185).  Plain 256-wide towers only up to
+        8192 rows, where the layers' GEMMs overtake its 16-row chains (3 x 256
+        relu on 300 inputs: 115 -> 104 us at 8192, 149 -> 156 at 12288)."""
         prog = self.prog
         A, C = prog.actor_layers, prog.critic_layers
         if (self.bf16 or prog.shared_head or not A or len(A) != len(C) or len(A) > lib.ppo_step_towers_max_layers()
@@ -114,7 +117,7 @@ class StepExecutor(ForwardChain):
             return False
         s0 = A[0]
         F, ln = s0.fout, s0.ln is not None
-        if (F not in ((256,) if ln else (64, 128, 256))
+        if (F not in ((256,) if ln else (64, 128, 256)) or (F == 256 and not ln and self.rows > 8192)
                 or s0.act not in ("relu", "tanh", None) + (("silu",) if ln else ())):
             return False
         for layers in (A, C):

@@ -178,6 +178,15 @@ def test_plain_towers_leave_their_one_launch_update_past_its_rounds(width, depth
         assert names.count("ppo_head_loss_f32") == int(not chain)
 
 
+@pytest.mark.parametrize("width, rows, joined", [(256, 8192, True), (256, 8193, False), (128, 65536, True), (64, 65536, True)])
+def test_plain_256_wide_towers_step_layer_by_layer_past_8192_rows(width, rows, joined):
+    from boonta_amd.rollout import StepExecutor
+    prog = tower_program(width, 1, 8)
+    ex = StepExecutor(prog, FlatState(prog, torch.device("cpu")), rows)
+    names = [n for n, _ in ex.record(4096, 8, 1.0, 16384, 20480, 24576)]
+    assert (names == ["ppo_step_towers_f32"]) == joined
+
+
 def test_shared_heads_pack_logits_and_value_in_one_matrix():
     r = recipes.make(2)
     prog = Program(r.network.plan(r.obs_dim))
