@@ -399,21 +399,37 @@ class ForwardChain:
         self.inp: dict = {}
 
     @staticmethod
-    def _f32_tile(a_layout: int, b_layout: int, M: int, K: int) -> int:
-        """fp32 tile for a whole-minibatch contraction (every tile of one
-        problem forms the same bits).  From 32768 rows (the Anakin minibatch)
-        the 8-wave 256 x 128 tile for forwards (32768 x 256 x 400: 47 us, 61 on
-        64 x 64) and 64 x 128 for the weight gradient of a 256-row kernel (38
-        us against 42; 128 x 128 the same); from 16384 rows 64 x 128 for the
-        input cotangents (B = W^T; 32768 x 256 x 256: 41 us against 44,
-        16384 x 256 x 768: 52 against 61).  Smaller minibatches and every other
-        shape: the library's default 64 x 64, whose grid fills more CUs."""
-        if a_layout == A_ROW and b_layout == B_KN and M >= 32768:
-            return 9
-        if a_layout == A_ROW and b_layout == B_NK and M >= 16384:
-            return 2
+    def _f32_tile(a_layout: int, b_layout: int, M: int, N: int, K: int, splits: int = 1) -> int:
+        """fp32 tile of one contraction (-1: the library's 64 x 64, whose grid
+        fills the CUs soonest), the lines set where alone-timed launches cross.
+
+        A wide tile pays where it pads no more columns than 64 x 64 would and
+        its grid fills its rounds.  Forwards, 256 x 128 on 8 waves, one
+        workgroup per CU, five sixths of a round: 32768 x 256 x 256 38 us (64 x
+        64 tiles 46), 64303 x 256 x 512 128 (157); 16384 x 256, half a round, 35
+        (26); 36786 x 512, 2.25 rounds, 100 (93); 32768 x 192, a quarter
+        padding, 39 (37).  Input cotangents (B = W^T), 64 x 128, two per CU,
+        three quarters, a contraction of 96 or more: 32768 x 256 x 256 41 us
+        (48), 41411 x 384 x 512 142 (155); 17515 x 256, 1.07 rounds, 50 (46);
+        32768 x 64, half padding, 10 (8); 16384 x 256 x 64 16 (12).  Over 72
+        shapes drawn from 4096 to 80000 rows and 72 to 1024 columns the choice
+        is within 6 % of the better tile (39315 x 300: 10 %).
+        Weight gradients of a 256-row kernel
+        over 32768 rows or more: 64 x 128 for 256 columns (43 us, 45), else
+        128 x 128 where it pads nothing and two of its workgroups per CU take
+        the whole grid (512 columns: 75, 85; 768, 516 workgroups: 163, 135)."""
+        tiles = lambda bm, bn: math.ceil(M / bm) * math.ceil(N / bn)
+        unpadded = math.ceil(N / 128) * 2 == math.ceil(N / 64)  # 128-wide columns pad as 64-wide ones do
+        if a_layout == A_ROW and b_layout == B_KN and unpadded:
+            t = tiles(256, 128)
+            return 9 if 6 * t >= 5 * 256 * math.ceil(t / 256) else -1
+        if a_layout == A_ROW and b_layout == B_NK and unpadded and K >= 96:
+            t = tiles(64, 128)
+            return 2 if 4 * t >= 3 * 512 * math.ceil(t / 512) else -1
         if a_layout == A_COL and M == 256 and K >= 32768:
-            return 2
+            if N == 256:
+                return 2
+            return 0 if N % 128 == 0 and tiles(128, 128) * splits <= 512 else -1
         return -1
 
     def _gemm(self, st, a_layout, b_layout, A, lda, rows, B, ldb, C, ldc, M, N, K, splits, stride, epi, bias, act,
@@ -424,7 +440,7 @@ class ForwardChain:
         fp32 and rounded after their sum)."""
         if not self.bf16:
             if tile == -1:
-                tile = self._f32_tile(a_layout, b_layout, M, K)
+                tile = self._f32_tile(a_layout, b_layout, M, N, K, splits)
             self._call("ppo_gemm_f32", st, a_layout, b_layout, A, lda, rows, B, ldb, C, ldc, M, N, K, splits, stride,
                        epi, bias, act, pre, aux, ldaux, bias_grad, tile)
             return

@@ -147,6 +147,21 @@ def test_flat_layout_round_trips_the_parameter_tree(config):
     assert prog.layout.size % 64 == 0
 
 
+@pytest.mark.parametrize("layouts, M, N, K, splits, tile", [
+    ("fwd", 32768, 256, 256, 1, 9), ("fwd", 32768, 200, 64, 1, 9), ("fwd", 16384, 512, 512, 1, 9),
+    ("fwd", 16384, 256, 400, 1, -1), ("fwd", 36786, 512, 256, 1, -1),        # half a round, 2.25 rounds
+    ("fwd", 32768, 192, 256, 1, -1), ("fwd", 131072, 64, 64, 1, -1), ("fwd", 65536, 8, 256, 1, -1),   # padding
+    ("dx", 32768, 256, 256, 1, 2), ("dx", 16384, 256, 768, 1, 2), ("dx", 32768, 96, 96, 1, 2),
+    ("dx", 17515, 256, 400, 1, -1), ("dx", 16384, 128, 768, 1, -1), ("dx", 16384, 256, 64, 1, -1),
+    ("dx", 32768, 64, 64, 1, -1), ("dx", 65536, 32, 32, 1, -1), ("dx", 12000, 300, 300, 1, -1),
+    ("dw", 256, 256, 32768, 64, 2), ("dw", 256, 512, 32768, 64, 0), ("dw", 256, 128, 65536, 256, 0),
+    ("dw", 256, 64, 32768, 256, -1), ("dw", 256, 768, 32768, 43, -1), ("dw", 256, 256, 16384, 128, -1)])
+def test_wide_tiles_are_chosen_where_their_grid_fills_without_padding(layouts, M, N, K, splits, tile):
+    from boonta_amd.learner import A_COL, A_ROW, B_KN, B_NK, ForwardChain
+    a, b = {"fwd": (A_ROW, B_KN), "dx": (A_ROW, B_NK), "dw": (A_COL, B_KN)}[layouts]
+    assert ForwardChain._f32_tile(a, b, M, N, K, splits) == tile
+
+
 class ActChainExecutor(MLPExecutor):
     CHAIN_ACT = True  # (on host memory too)
 
