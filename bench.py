@@ -427,7 +427,7 @@ def time_launches(ex, reps, per_update_steps):
         e1.synchronize()
         flops, nbytes = launch_work(name, args)
         row = {"i": i, "name": name, "ms_alone": e0.elapsed_time(e1) / reps, "count": count, "flops": flops,
-               "bytes": nbytes, "shape": launch_shape(name, args), "layout": launch_layout(name, args),
+               "peak": mfma_peak(name, args), "bytes": nbytes, "shape": launch_shape(name, args), "layout": launch_layout(name, args),
                "ctx": []}
         rows.append(row)
         seen[key] = row
@@ -569,8 +569,22 @@ def _cpu_baseline_pupo(recipe, params, plan, cfg, opt, key, budget_s, tr):
 BF16_KERNELS = ("ppo_gemm_bf16", "ppo_gemm_bf16s", "ppo_gemm_bf16s_dw_group", "ppo_mlp16_ln_fwd", "ppo_mlp16_ln_bwd")
 
 
+def mfma_peak(name, args):
+    """TFLOP/s of the matrix instructions a launch runs on: bf16 ones, fp32
+    ones, or fp32 products as eight bf16 ones each (the wide tiles of
+    ppo_gemm_f32's row layouts, where every operand row takes 16-byte loads)."""
+    if name in BF16_KERNELS:
+        return PEAK["bf16_mfma"]
+    base, a, _ = untower(name, args)
+    if base == "ppo_gemm_f32" and a[1] == 0 and a[22] in (2, 8, 9):
+        A, lda, B, ldb, N, K = a[3], a[4], a[6], a[7], a[11], a[12]
+        if not any(x % 4 for x in (lda, ldb, K, K if a[2] else N)) and not (A % 16 or B % 16):
+            return PEAK["bf16_mfma"] / 8
+    return PEAK["fp32_mfma"]
+
+
 def roofline_of(dom, total, workload):
-    peak = PEAK["bf16_mfma"] if dom["name"] in BF16_KERNELS else PEAK["fp32_mfma"]
+    peak = dom["peak"]
     # the roof the kernel meets first: its MFMA time at peak against its HBM time at peak
     if dom["flops"] > 0 and dom["flops"] / (peak * 1e12) >= dom["bytes"] / (PEAK["hbm"] * 1e9):
         achieved = dom["flops"] / (dom["ms"] * 1e-3) / 1e12
@@ -598,7 +612,7 @@ def launch_rows(rows):
     for r in rows:
         e = {k: r[k] for k in ("name", "layout", "shape", "ms", "ms_bracketed", "ms_alone", "count") if k in r}
         sec = r["ms"] * 1e-3
-        peak = PEAK["bf16_mfma"] if r["name"] in BF16_KERNELS else PEAK["fp32_mfma"]
+        peak = r["peak"]
         # the roof a launch meets first: its MFMA time at peak against its HBM time at peak
         if r["flops"] > 0 and r["flops"] / (peak * 1e12) >= r["bytes"] / (PEAK["hbm"] * 1e9):
             e.update(bound="mfma", achieved=r["flops"] / sec / 1e12, frac=r["flops"] / sec / 1e12 / peak)
@@ -683,7 +697,7 @@ def time_calls(calls, reps, count):
         e1.record(stream)
         e1.synchronize()
         flops, nbytes = launch_work(name, args)
-        row = {"i": i, "name": name, "ms": e0.elapsed_time(e1) / reps, "count": count, "flops": flops,
+        row = {"i": i, "name": name, "ms": e0.elapsed_time(e1) / reps, "count": count, "flops": flops, "peak": mfma_peak(name, args),
                "bytes": nbytes, "shape": launch_shape(name, args), "layout": launch_layout(name, args)}
         rows.append(row)
     return rows

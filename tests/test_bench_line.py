@@ -58,3 +58,22 @@ def test_headline_line_is_short_and_complete(capsys, tmp_path):
     d = json.loads(detail.read_text())
     assert len(d["headline"]["launches"]) == 40 and len(d["configs"]) == 4
     assert "[bench] detail " in captured.err
+
+
+def test_each_launch_is_held_against_the_matrix_instructions_it_runs_on():
+    gemm = lambda al, bl, tile, lda=256, A=4096, N=256, K=256: (
+        0, al, bl, A, lda, None, 8192, 256, 1 << 20, N, 32768, N, K, 1, 0, 0, None, 0, None, None, 0, None, tile)
+    fp32, bf16 = bench.PEAK["fp32_mfma"], bench.PEAK["bf16_mfma"]
+    assert bench.mfma_peak("ppo_gemm_f32", gemm(0, 0, 9)) == bf16 / 8    # split products
+    assert bench.mfma_peak("ppo_gemm_f32", gemm(0, 1, 2)) == bf16 / 8
+    for args in (gemm(0, 0, -1), gemm(0, 0, 0), gemm(1, 0, 2), gemm(0, 0, 9, lda=257), gemm(0, 0, 9, A=4100)):
+        assert bench.mfma_peak("ppo_gemm_f32", args) == fp32
+    towers = gemm(0, 1, 2)
+    assert bench.mfma_peak("ppo_gemm_f32_towers", (0, 2) + towers[1:] + (0,) * 7) == bf16 / 8
+    assert bench.mfma_peak("ppo_gemm_bf16s", ()) == bf16 and bench.mfma_peak("ppo_mlp_ln_fwd_f32", (0,) * 30) == fp32
+    # a split launch's share of its peak, and the roof it meets first
+    row = {"name": "ppo_gemm_f32", "layout": [0, 0], "shape": [32768, 256, 256], "ms": 0.038, "count": 64,
+           "flops": 2.0 * 32768 * 256 * 256, "bytes": 4.0 * 2 * 32768 * 256, "peak": bf16 / 8}
+    roof = bench.roofline_of(row, 8.0, "none")
+    assert roof["bound"] == "mfma" and roof["peak"] == bf16 / 8 and 0.3 < roof["frac"] < 0.4
+    assert bench.launch_rows([row])[0]["frac"] == roof["frac"]
