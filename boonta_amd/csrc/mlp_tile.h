@@ -8,7 +8,6 @@ namespace {
 template <int NB> struct VecOf;
 template <> struct VecOf<1> { typedef float type; };
 template <> struct VecOf<2> { typedef float type __attribute__((ext_vector_type(2))); };
-template <> struct VecOf<4> { typedef floatx4 type; };
 
 template <int NB>
 __device__ __forceinline__ void load_nb(const float* p, float (&v)[NB]) {

@@ -358,8 +358,8 @@ def paired_tower_bufs(specs_a, specs_c, rows: int, device, ln_blocks: int | None
         # split-K sums (the last split of each tile reads the others'
         # partials back), fewer splits: 3/4 for the first layer, half for the
         # later ones (2048-row minibatches, 12 and 8 splits: 2-layer tanh towers
-        # 2227 us per update of 32, 8 / 6 splits 2293, 16 / 12 2248; 4-layer
-        # LayerNorm towers 3199, 3210, 3268)
+        # 2138 us per update of 32, 8 / 6 splits 2246, 16 / 12 2173; 4-layer
+        # LayerNorm towers 3338, 3329, 3465)
         sp = _splits(rows, s.dense.fin, s.ld)
         if grouped_dw:
             # (a count the launch's finishing sums are compiled for)

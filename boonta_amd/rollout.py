@@ -261,7 +261,8 @@ class RecurrentStepExecutor(ForwardChain):
         self.head_samples = fused and _head_samples(program, lib)
         if not self.input_proj:
             self.XI = torch.zeros(rows, 3 * H, **f32)
-        self.HEAD = torch.zeros(rows, program.head_a.w.ld, **f32)
+        if not self.head_samples:
+            self.HEAD = torch.zeros(rows, program.head_a.w.ld, **f32)
         self.KEY = torch.zeros(2, dtype=torch.int32, device=dev)
 
     def issue(self, st: int, obs: int, ldo: int, carry: int, terminated: int | None, truncated: int | None,
