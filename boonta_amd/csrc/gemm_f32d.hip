@@ -342,7 +342,7 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
     } else {
       // a 16-deep block of the reduction (two groups per lane half); the next
       // block's LDS reads are issued once this block's operands are split,
-      // ahead of its products
+      // ahead of its last products (one A fragment at a time: two spilled)
       floatx4 a4[2][MB], b4[2][NB];
       auto read_ops = [&](int blk) {
 #pragma unroll
@@ -358,21 +358,21 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
       read_ops(0);
 #pragma unroll
       for (int blk = 0; blk < BK / 16; ++blk) {
-        ppo::Split8 fa[MB], fb[NB];
-#pragma unroll
-        for (int bi = 0; bi < MB; ++bi) fa[bi] = ppo::split8(a4[0][bi], a4[1][bi]);
+        ppo::Split8 fa = ppo::split8(a4[0][0], a4[1][0]), fb[NB];
 #pragma unroll
         for (int bj = 0; bj < NB; ++bj) fb[bj] = ppo::split8(b4[0][bj], b4[1][bj]);
-        if (blk + 1 < BK / 16) read_ops(blk + 1);
 #pragma unroll
-        for (int t = 0; t < ppo::SPLIT_PRODUCTS; ++t)
+        for (int bi = 0; bi < MB; ++bi) {
+          if (bi) fa = ppo::split8(a4[0][bi], a4[1][bi]);
+          if (bi == MB - 1 && blk + 1 < BK / 16) read_ops(blk + 1);
 #pragma unroll
-          for (int bi = 0; bi < MB; ++bi)
+          for (int t = 0; t < ppo::SPLIT_PRODUCTS; ++t)
 #pragma unroll
             for (int bj = 0; bj < NB; ++bj) {
               floatx16& c = t + 1 < ppo::SPLIT_PRODUCTS ? low[bi][bj] : acc[bi][bj];
-              c = ppo::split_mfma(t, fa[bi], fb[bj], c);
+              c = ppo::split_mfma(t, fa, fb[bj], c);
             }
+        }
       }
     }
   }
@@ -412,7 +412,8 @@ __device__ __forceinline__ void gemm_f32d_tile(const GemmParams& p, int tm, int 
 }
 
 template <int BM, int BN, int WM, int WN, bool A_K, bool B_K, int NBUF, bool SPLIT>
-__global__ void __launch_bounds__(WM * WN * 64, 2) gemm_f32d_kernel(GemmParams p0) {
+__global__ void __launch_bounds__(WM * WN * 64, SPLIT && BM * BN / (WM * WN) == 2048 ? 3 : 2)
+    gemm_f32d_kernel(GemmParams p0) {
   const ppo::TileCoord tc = ppo::xcd_tile();
   const int tower = tc.z / p0.splits;
   const int split = tc.z - tower * p0.splits;
