@@ -378,7 +378,9 @@ int ppo_ssm_scan_bwd(void* stream, int dtype, const void* a, const void* h, cons
  *   tile: -1 automatic (64x64); 0 128x128, 1 128x64, 2 64x128, 3 64x64
  *   (operands copied straight into LDS, 32 reduction steps per stage); 4-7
  *   the same tiles staged through registers; 8 128x256, 9 256x128 (8 waves,
- *   copied straight into LDS). */
+ *   copied straight into LDS).  a_layout 0 on copied tiles 2, 8 and 9: products
+ *   of three bf16 pieces a value (every bit kept); the others fp32 MFMA, whose
+ *   sums differ in rounding. */
 int ppo_gemm_f32(void* stream, int a_layout, int b_layout, const float* A, int64_t lda, const int32_t* rows,
                  const float* B, int64_t ldb, float* C, int64_t ldc, int M, int N, int K, int splits,
                  int64_t c_split_stride, int epi, const float* bias, int act, float* pre, const float* aux,

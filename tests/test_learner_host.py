@@ -193,6 +193,19 @@ def test_plain_towers_leave_their_one_launch_update_past_its_rounds(width, depth
         assert names.count("ppo_head_loss_f32") == int(not chain)
 
 
+def test_inputs_past_the_launchs_32_bit_offsets_are_left_to_the_layers():
+    from dataclasses import replace
+    from types import SimpleNamespace
+    r = recipes.make(1)
+    prog = tower_program(64, 1, 8)
+    ex = ActChainExecutor(prog, FlatState(prog, torch.device("cpu")), r.cfg, r.optimizer, 1, 32)
+    lead = prog.actor_layers[0]
+    for fin, chain in ((2 ** 25 - 1, True), (2 ** 25, False)):
+        wide = replace(lead, dense=replace(lead.dense, fin=fin))
+        p = SimpleNamespace(actor_layers=[wide], head_a=prog.head_a, head_c=prog.head_c)
+        assert ex._act_chainable(p, 32) == chain
+
+
 @pytest.mark.parametrize("width, rows, joined", [(256, 8192, True), (256, 8193, False), (128, 65536, True), (64, 65536, True)])
 def test_plain_256_wide_towers_step_layer_by_layer_past_8192_rows(width, rows, joined):
     from boonta_amd.rollout import StepExecutor
