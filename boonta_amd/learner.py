@@ -1333,8 +1333,8 @@ class MLPExecutor(ForwardChain):
         """Back-propagates through layers whose last output cotangent is in
         place, on one stream: a later layer's weight gradient beside its input
         cotangent gained 0.3 % at 65536 x 512 x 512 multiply-adds and cost 5-18
-        % at small minibatches, and a replay of such a graph (three layers, two
-        branches a step) ended in a host fault whose cause is not known."""
+        % at small minibatches, and replays of such graphs (two branches in all)
+        ended in a host fault twice, the cause not known."""
         c = layers[0].chain16 if layers else None
         if c is not None and c["bwd"]:
             # every LayerNorm backward and input cotangent in one launch; then
@@ -1910,10 +1910,16 @@ class MLPExecutor(ForwardChain):
         return calls
 
     # ------------------------------------------------------ two towers at once
+    # Updates of fewer optimizer steps stay on one stream.  Two replays of a
+    # captured update with side-stream branches have ended in a host fault whose
+    # cause is not known; both graphs had exactly two branches (what unequal
+    # towers have in one step), where graphs of four and more have run throughout.
+    SIDE_STEPS = 4
+
     def _fork(self, st: int) -> int:
         """Handle of the side stream, ordered after everything issued on st so
         far (inside a graph capture this forks the captured graph)."""
-        if self._recording or self.side is None:
+        if self._recording or self.side is None or self.E * self.M < self.SIDE_STEPS:
             return st
         side = self.side.cuda_stream
         if st == side:

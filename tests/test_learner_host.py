@@ -125,6 +125,30 @@ def test_a_shared_trunk_update_stays_on_one_stream():
     assert {args[0] for _, args in calls} == {7}
 
 
+@pytest.mark.parametrize("epochs, minibatches, branches", [(1, 1, 0), (1, 2, 0), (1, 4, 8), (2, 2, 8)])
+def test_unequal_towers_take_the_side_stream_from_four_steps_on(epochs, minibatches, branches):
+    """(one branch in each direction of a step, forked and joined)"""
+    from dataclasses import replace
+    from types import SimpleNamespace
+    from boonta_amd import networks as nn
+    torso = lambda w: [nn.Dense(w), nn.tanh]
+    net = nn.Network(feature_extractor=nn.FeatureExtractor(nn.Identity()),
+                     head=nn.ActorCritic(actor=nn.Categorical(nn.Sequential(torso(64) + [nn.Dense(6)])),
+                                         critic=nn.Sequential(torso(32) + [nn.Dense(1)])))
+    r = recipes.make(1)
+    cfg = replace(r.cfg, num_minibatches=minibatches, update_epochs=epochs)
+    prog = Program(net.plan(8))
+    ex = MLPExecutor(prog, FlatState(prog, torch.device("cpu")), cfg, r.optimizer, 4, 16)
+    assert not ex.pair
+    ex.side, ex._ev_fork, ex._ev_join = SimpleNamespace(cuda_stream=99), 1, 2
+    ex.bind(fake_inputs(ex))
+    calls = []
+    ex._call = lambda name, *args: calls.append((name, args))
+    ex.issue(7)
+    assert [n for n, _ in calls].count("ppo_stream_wait") == 2 * branches
+    assert {args[0] for _, args in calls} == ({7, 99} if branches else {7})
+
+
 @pytest.mark.parametrize("config", ALL_CONFIGS)
 def test_flat_layout_round_trips_the_parameter_tree(config):
     r = recipes.make(config)
