@@ -17,6 +17,8 @@ buffers are updated in place and the returned state shares them.
 """
 from __future__ import annotations
 
+import gc
+import threading
 from dataclasses import dataclass, field
 from typing import Any, Callable
 
@@ -73,6 +75,32 @@ def _first_leaf(tree):
     while isinstance(tree, dict):
         tree = tree[sorted(tree)[0]]
     return tree
+
+
+_CAPTURE = threading.Lock()  # (the collector's state is the process's)
+
+
+def capture(issue) -> torch.cuda.CUDAGraph:
+    """The launches of ``issue(stream handle)`` as a HIP graph.  Python's cyclic
+    collector is held off meanwhile: a dropped state, its executors and their
+    graphs form a cycle, so it is the collector that destroys them, at any
+    allocation, and a graph's destructor waits for the device, which no thread
+    may do while a stream is capturing (the process ended there)."""
+    g = torch.cuda.CUDAGraph()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with _CAPTURE:
+        collecting = gc.isenabled()
+        gc.disable()
+        try:
+            with torch.cuda.stream(side):
+                with torch.cuda.graph(g, stream=side):
+                    issue(torch.cuda.current_stream().cuda_stream)
+        finally:
+            if collecting:
+                gc.enable()
+    torch.cuda.current_stream().wait_stream(side)
+    return g
 
 
 @dataclass
@@ -281,13 +309,7 @@ class PPO:
             for dst, src in zip((flat.P, flat.MU, flat.NU, flat.count), snapshot):
                 dst.copy_(src)
             torch.cuda.synchronize()
-            g = torch.cuda.CUDAGraph()
-            side = torch.cuda.Stream()
-            side.wait_stream(torch.cuda.current_stream())
-            with torch.cuda.stream(side):
-                with torch.cuda.graph(g, stream=side):
-                    ex.issue(torch.cuda.current_stream().cuda_stream)
-            torch.cuda.current_stream().wait_stream(side)
+            g = capture(ex.issue)
             while len(ex.graphs) >= self.MAX_GRAPHS:
                 ex.graphs.pop(next(iter(ex.graphs)))
             ex.graphs[gk] = g

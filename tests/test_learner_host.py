@@ -676,3 +676,53 @@ def test_recurrent_update_runs_each_direction_of_the_recurrence_in_one_launch(fu
             assert args[25] == ex.SEQX.data_ptr()
             assert args[36:] == ((1, ex.SEQX_F.data_ptr(), 8 * ex.SEQX_F.numel()) if pair else (0, None, 0))
             assert ex.wh_splits == ex.wi_splits == (Bm + 15) // 16 == ex.WHPART.shape[0] == ex.WIPART.shape[0]
+
+
+def test_no_collection_falls_into_a_capture(monkeypatch):
+    """What dropped states leave behind (a cycle of state, executors and graphs,
+    whose destructors wait for the device) is not collected while a stream
+    captures, and is afterwards."""
+    import contextlib
+    import gc
+    from types import SimpleNamespace
+    from boonta_amd.algorithms import ppo
+
+    capturing, collected = [], []
+
+    class Dropped:
+        def __init__(self):
+            self.me = self
+
+        def __del__(self):
+            collected.append(bool(capturing))
+
+    @contextlib.contextmanager
+    def graph(g, stream):
+        capturing.append(g)
+        yield
+        capturing.pop()
+
+    stream = SimpleNamespace(cuda_stream=7, wait_stream=lambda s: None)
+    for name, fake in (("CUDAGraph", object), ("Stream", lambda: stream), ("current_stream", lambda: stream),
+                       ("stream", lambda s: contextlib.nullcontext()), ("graph", graph)):
+        monkeypatch.setattr(torch.cuda, name, fake)
+
+    def issue(st):
+        assert st == 7 and capturing
+        for _ in range(5):
+            Dropped()
+            [[] for _ in range(2000)]   # (allocations enough to start a collection)
+
+    thresholds = gc.get_threshold()
+    try:
+        gc.set_threshold(100, 1, 1)
+        ppo.capture(issue)
+        assert gc.isenabled()
+        gc.collect()
+        with pytest.raises(RuntimeError), monkeypatch.context() as m:
+            m.setattr(torch.cuda, "graph", lambda g, stream: (_ for _ in ()).throw(RuntimeError("refused")))
+            ppo.capture(issue)
+        assert gc.isenabled()
+    finally:
+        gc.set_threshold(*thresholds)
+    assert collected == [False] * 5
