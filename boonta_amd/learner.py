@@ -913,7 +913,7 @@ class MLPExecutor(ForwardChain):
         """Towers ppo_mlp_act_fwd_head_loss_bwd_f32 takes: up to
         ppo_mlp_chain_max_layers() Dense(F) layers (F = 64, 128 or 256) of one
         activation (relu, tanh or none) and no LayerNorm under the fused heads,
-        and a minibatch within _act_chain_rows."""
+        where that is faster (_act_chain_faster)."""
         layers, lib = program.actor_layers, _lib.load()
         if not (self.flat.P.is_cuda if self.CHAIN_ACT is None else self.CHAIN_ACT):
             return False
@@ -926,8 +926,7 @@ class MLPExecutor(ForwardChain):
         if any(s.ln is not None or s.fout != F or s.ld != F or s.dense.w.ld != F or s.act != s0.act
                or (i > 0 and s.dense.fin != F) for i, s in enumerate(layers)):
             return False
-        K0 = s0.dense.fin
-        if mb > self._act_chain_rows(F, K0, len(layers)) or K0 * F > 2 ** 31 - 1:
+        if not self._act_chain_faster(F, s0.dense.fin, len(layers), mb):
             return False
         # the launch copies each head kernel into LDS from its 256-byte aligned start
         base = self.flat.P.data_ptr() if self.flat.P.is_cuda else 0
@@ -936,21 +935,32 @@ class MLPExecutor(ForwardChain):
                 and lib.ppo_head_loss_blocks(mb) == -(-mb // 16))
 
     @staticmethod
-    def _act_chain_rows(F: int, K0: int, L: int) -> int:
-        """Largest minibatch of the plain towers' launch.  A round of its
-        workgroups (16 rows of one tower each) takes as long as one, where the
-        layers' own launches grow with the rows; it saves their count.  One round
-        (one workgroup per CU, two of 64 wide) is faster always, two where
-        several layers are saved and a row's products are few; us an update of
-        8 steps, this launch and layer by layer:
+    def _act_chain_faster(F: int, K0: int, L: int, rows: int) -> bool:
+        """Whether the plain towers' launch beats the layers' own for a minibatch
+        (us an update of 8 steps, this launch / layer by layer).
+
+        A round of its workgroups (16 rows of one tower each) takes as long as
+        one, where the layers' own launches grow with the rows; it saves their
+        count.  One round (one workgroup per CU, two of 64 wide) gains, two where
+        several layers are saved and a row's products are few:
           64 wide: 1 layer on 20 inputs, 4096 rows 327 / 348, 8192 414 / 406;
             3 on 376, 8192 780 / 870, 12288 1137 / 1063
           128: 1 on 87, 2048 348 / 387, 3072 436 / 413; 3 on 376, 4096
             807 / 839, 6144 1146 / 1089
           256: 1 on 20, 2048 365 / 419, 3072 484 / 457; 2 on 87, 4096 930 /
-            958, 6144 1311 / 1206; 3 on 376, 2048 957 / 1048, 3072 1533 / 1353."""
+            958, 6144 1311 / 1206; 3 on 376, 2048 957 / 1048, 3072 1533 / 1353.
+        A wide input's kernel is a long chain of loads for every workgroup, the
+        longer where too few of them share it to bring it into L2 first (below
+        512 rows); the layers' GEMMs spread its columns over the CUs:
+          128 rows: 128 wide, 1 layer on 325 378 / 481, on 600 464 / 452; 256
+            wide, 1 on 87 363 / 417, on 325 571 / 517; 2 on 325 735 / 771, on
+            600 954 / 744; 3 on 325 906 / 1020, on 600 1121 / 1005
+          1024 rows, 256 wide: 1 on 325 557 / 608, on 600 686 / 628; 2 on
+            600 885 / 878; 3 on 600 1043 / 1131."""
+        if K0 * F > (100_000 if rows >= 512 else 42_000) * L:
+            return False
         rounds = 2 if L > 1 and F * (K0 + 2 * (L - 1) * F) <= 160_000 else 1
-        return rounds * (4096 if F == 64 else 2048)
+        return rows <= rounds * (4096 if F == 64 else 2048)
 
     def _act_tables(self):
         """Per-layer pointer tables of the plain towers' launch (kept alive on

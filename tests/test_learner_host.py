@@ -217,17 +217,21 @@ def test_plain_towers_leave_their_one_launch_update_past_its_rounds(width, depth
         assert names.count("ppo_head_loss_f32") == int(not chain)
 
 
-def test_inputs_past_the_launchs_32_bit_offsets_are_left_to_the_layers():
+@pytest.mark.parametrize("width, depth, obs, rows, chain", [
+    (256, 1, 164, 128, True), (256, 1, 165, 128, False), (256, 1, 390, 512, True), (256, 1, 391, 512, False),
+    (128, 1, 328, 32, True), (128, 1, 329, 32, False), (256, 2, 325, 128, True), (256, 2, 600, 128, False),
+    (256, 2, 600, 1024, True), (256, 3, 600, 256, False), (64, 1, 2 ** 26, 32, False)])
+def test_wide_inputs_are_left_to_the_layers_where_their_kernel_is_a_long_chain(width, depth, obs, rows, chain):
+    """(2^26 inputs: past the launch's 32-bit offsets as well)"""
     from dataclasses import replace
     from types import SimpleNamespace
     r = recipes.make(1)
-    prog = tower_program(64, 1, 8)
+    prog = tower_program(width, depth, 8)
     ex = ActChainExecutor(prog, FlatState(prog, torch.device("cpu")), r.cfg, r.optimizer, 1, 32)
     lead = prog.actor_layers[0]
-    for fin, chain in ((2 ** 25 - 1, True), (2 ** 25, False)):
-        wide = replace(lead, dense=replace(lead.dense, fin=fin))
-        p = SimpleNamespace(actor_layers=[wide], head_a=prog.head_a, head_c=prog.head_c)
-        assert ex._act_chainable(p, 32) == chain
+    wide = replace(lead, dense=replace(lead.dense, fin=obs))
+    p = SimpleNamespace(actor_layers=[wide] + prog.actor_layers[1:], head_a=prog.head_a, head_c=prog.head_c)
+    assert ex._act_chainable(p, rows) == chain
 
 
 @pytest.mark.parametrize("width, rows, joined", [(256, 8192, True), (256, 8193, False), (128, 65536, True), (64, 65536, True)])
