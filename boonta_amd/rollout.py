@@ -104,12 +104,20 @@ class StepExecutor(ForwardChain):
         return {"keep": keep, "args": (n, *map(ctypes.addressof, keep), _act(prog.trunk[0].act), view(h.w), h.w.ld)}
 
     def _towers_fusable(self, lib) -> bool:
-        """Whether the paired towers' one-launch step covers this program: it
-        replaces two launches per layer and three after (4 x 256 LayerNorm +
-        SiLU, 4096 rows: 125 -> 64 us, 65536: 1144 -> 937; 2 x 64 and 2 x 128
-        tanh, 65536: 150 -> 67 and 207 -> 185).  Plain 256-wide towers only up to
-        8192 rows, where the layers' GEMMs overtake its 16-row chains (3 x 256
-        relu on 300 inputs: 115 -> 104 us at 8192, 149 -> 156 at 12288)."""
+        """Whether the paired towers' one-launch step covers this program, and
+        its number of rows: it replaces two launches per layer and three after (4
+        x 256 LayerNorm + SiLU, 4096 rows: 125 -> 64 us).  The layers' GEMMs
+        overtake its 16-row chains on fp32 MFMA as the rows' products grow beside
+        the launches saved, sooner where the input's rows take no 16-byte loads.
+        Us, this launch / layer by layer: plain towers, 3 x 256 on 300 inputs,
+        9000 rows 136 / 165, 12288 156 / 149; 2 x 256 on 87, 16384 109 / 120; 1 x
+        256 on 600, 4096 52 / 67, on 1000, 7000 159 / 117; 1 x 128 on 600, 4096
+        36 / 60, 16384 157 / 81, on 159, 10580 70 / 52; 4 x 64 on 98, 52037 154 /
+        154.  With LayerNorm, whose layers run 16-row tiles as well, only through
+        a wide input: 4 x 256 on 87, 65536 rows 937 / 1144; 1 x 256 on 916, 2994
+        75 / 87, on 1500, 16384 456 / 406, on 489, 7020 157 / 129, on 109,
+        48756 239 / 190; 2 x 256 on 2044, 11341 500 / 563, on 2010, 856 292 / 220.
+        Over 83 drawn shapes the choice is within 14 % of the better."""
         prog = self.prog
         A, C = prog.actor_layers, prog.critic_layers
         if (self.bf16 or prog.shared_head or not A or len(A) != len(C) or len(A) > lib.ppo_step_towers_max_layers()
@@ -117,7 +125,7 @@ class StepExecutor(ForwardChain):
             return False
         s0 = A[0]
         F, ln = s0.fout, s0.ln is not None
-        if (F not in ((256,) if ln else (64, 128, 256)) or (F == 256 and not ln and self.rows > 8192)
+        if (F not in ((256,) if ln else (64, 128, 256))
                 or s0.act not in ("relu", "tanh", None) + (("silu",) if ln else ())):
             return False
         for layers in (A, C):
@@ -125,6 +133,16 @@ class StepExecutor(ForwardChain):
                 if (s.fout != F or s.ld != F or s.dense.w.ld != F or s.act != s0.act or (s.ln is not None) != ln
                         or s.dense.fin != (A[0].dense.fin if i == 0 else F) or (ln and s.ln["eps"] != s0.ln["eps"])):
                     return False
+        K0 = s0.dense.fin
+        L, aligned = len(A), K0 % 4 == 0
+        if ln:
+            wide = K0 * F > (280_000 if aligned else 60_000 if self.rows <= 16384 else 20_000) * L
+            if wide and (self.rows > 2048 or not aligned):
+                return False
+        else:
+            macs = self.rows * F * ((1.0 if aligned else 1.5) * K0 + (L - 1) * F)  # of one tower
+            if macs > ((0.5 + 0.5 * L) if F == 256 else (0.32 + 0.4 * (L - 1))) * 1e9:
+                return False
         ha, hc = prog.head_a, prog.head_c
         gaussian = prog.dist["kind"] != "categorical"
         if gaussian and (prog.scale_region is None or prog.dist["dim"] != prog.head_out):

@@ -234,12 +234,29 @@ def test_wide_inputs_are_left_to_the_layers_where_their_kernel_is_a_long_chain(w
     assert ex._act_chainable(p, rows) == chain
 
 
-@pytest.mark.parametrize("width, rows, joined", [(256, 8192, True), (256, 8193, False), (128, 65536, True), (64, 65536, True)])
-def test_plain_256_wide_towers_step_layer_by_layer_past_8192_rows(width, rows, joined):
+@pytest.mark.parametrize("width, depth, obs, rows, joined", [
+    (256, 1, 8, 65536, True), (256, 3, 300, 9000, True), (256, 3, 300, 12288, False), (256, 1, 600, 4096, True),
+    (256, 1, 1000, 7000, False), (128, 1, 600, 4096, True), (128, 1, 600, 16384, False), (64, 3, 600, 4096, True),
+    (64, 3, 600, 32768, False), (128, 1, 159, 10580, False), (128, 1, 160, 10580, True)])
+def test_plain_towers_step_layer_by_layer_past_their_launchs_products(width, depth, obs, rows, joined):
+    steps_in_one_launch(tower_program(width, depth, obs), obs, rows, joined)
+
+
+@pytest.mark.parametrize("depth, obs, rows, joined", [(1, 916, 2994, True), (1, 1500, 2048, True), (1, 1500, 2049, False),
+                                                      (2, 2044, 11341, True), (2, 2010, 856, False), (4, 87, 65536, True)])
+def test_layernorm_towers_step_layer_by_layer_on_wide_inputs(depth, obs, rows, joined):
+    from boonta_amd import networks as nn
+    torso = lambda: [f for _ in range(depth) for f in (nn.Dense(256), nn.LayerNorm(), nn.silu)]
+    net = nn.Network(feature_extractor=nn.FeatureExtractor(nn.Identity()),
+                     head=nn.ActorCritic(actor=nn.Categorical(nn.Sequential(torso() + [nn.Dense(6)])),
+                                         critic=nn.Sequential(torso() + [nn.Dense(1)])))
+    steps_in_one_launch(Program(net.plan(obs)), obs, rows, joined)
+
+
+def steps_in_one_launch(prog, obs, rows, joined):
     from boonta_amd.rollout import StepExecutor
-    prog = tower_program(width, 1, 8)
     ex = StepExecutor(prog, FlatState(prog, torch.device("cpu")), rows)
-    names = [n for n, _ in ex.record(4096, 8, 1.0, 16384, 20480, 24576)]
+    names = [n for n, _ in ex.record(4096, obs, 1.0, 16384, 20480, 24576)]
     assert (names == ["ppo_step_towers_f32"]) == joined
 
 
