@@ -275,7 +275,12 @@ class RecurrentStepExecutor(ForwardChain):
         f32 = dict(dtype=torch.float32, device=dev)
         self.rows = rows
         self.trunk: list[LayerBufs] = [forward_bufs(s, rows, dev) for s in program.trunk]
-        self.input_proj = fused and program.gru.fin % 64 == 0
+        # (ahead of the projection GEMM and the step apart at every size timed but
+        # wide inputs of many sequences: 1024 -> 256, 4096 120 / 115 us, 16384 404 /
+        # 369; 512 -> 64, 4096 30 / 38, 16384 78 / 71; 2048 -> 128 107 / 119, 373 /
+        # 325; 256 -> 512, 16384 480 / 551)
+        self.input_proj = (fused and program.gru.fin % 64 == 0
+                           and not (program.gru.fin >= 4 * H and rows > 4096))
         self.head_samples = fused and _head_samples(program, lib)
         if not self.input_proj:
             self.XI = torch.zeros(rows, 3 * H, **f32)

@@ -253,6 +253,20 @@ def test_layernorm_towers_step_layer_by_layer_on_wide_inputs(depth, obs, rows, j
     steps_in_one_launch(Program(net.plan(obs)), obs, rows, joined)
 
 
+@pytest.mark.parametrize("I, H, rows, joined", [(512, 64, 4096, True), (512, 64, 4097, False), (192, 64, 16384, True),
+                                                (256, 256, 65536, True), (96, 64, 16, False)])
+def test_recurrent_steps_form_the_projections_but_from_wide_inputs_of_many_sequences(I, H, rows, joined):
+    from boonta_amd import networks as nn
+    from boonta_amd.rollout import RecurrentStepExecutor
+    net = nn.Network(feature_extractor=nn.FeatureExtractor(nn.Sequential([nn.Dense(I), nn.relu])),
+                     torso=nn.RNN(nn.GRUCell(H)), head=nn.ActorCritic(actor=nn.Categorical(nn.Dense(4)),
+                                                                      critic=nn.Dense(1)))
+    prog = Program(net.plan(8))
+    ex = RecurrentStepExecutor(prog, FlatState(prog, torch.device("cpu")), rows, fused=True)
+    names = [n for n, _ in ex.record(4096, 8, 8192, 12288, 16384, 1.0, 20480, 24576, 28672, 32768)]
+    assert ("ppo_gru_fwd_step_x_f32" in names) == joined and ("ppo_gru_fwd_step_f32" in names) == (not joined)
+
+
 def steps_in_one_launch(prog, obs, rows, joined):
     from boonta_amd.rollout import StepExecutor
     ex = StepExecutor(prog, FlatState(prog, torch.device("cpu")), rows)
