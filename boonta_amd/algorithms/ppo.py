@@ -80,7 +80,26 @@ def _first_leaf(tree):
 _CAPTURE = threading.Lock()  # (the collector's state is the process's)
 
 
-def capture(issue) -> torch.cuda.CUDAGraph:
+class UpdateGraph:
+    """A captured update.  Its graph outlives it where it is collected while the
+    caller captures a graph of their own (a rollout of steps, say, after other
+    states were dropped): destroying one there ends the process, so it waits for
+    the next captured update."""
+
+    _held: list = []
+
+    def __init__(self, graph):
+        self.graph = graph
+
+    def replay(self):
+        self.graph.replay()
+
+    def __del__(self):
+        if torch is not None and torch.cuda.is_current_stream_capturing():
+            UpdateGraph._held.append(self.graph)
+
+
+def capture(issue) -> UpdateGraph:
     """The launches of ``issue(stream handle)`` as a HIP graph.  Python's cyclic
     collector is held off meanwhile: a dropped state, its executors and their
     graphs form a cycle, so it is the collector that destroys them, at any
@@ -90,6 +109,7 @@ def capture(issue) -> torch.cuda.CUDAGraph:
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with _CAPTURE:
+        UpdateGraph._held.clear()
         collecting = gc.isenabled()
         gc.disable()
         try:
@@ -100,7 +120,7 @@ def capture(issue) -> torch.cuda.CUDAGraph:
             if collecting:
                 gc.enable()
     torch.cuda.current_stream().wait_stream(side)
-    return g
+    return UpdateGraph(g)
 
 
 @dataclass

@@ -738,7 +738,8 @@ def test_no_collection_falls_into_a_capture(monkeypatch):
         capturing.pop()
 
     stream = SimpleNamespace(cuda_stream=7, wait_stream=lambda s: None)
-    for name, fake in (("CUDAGraph", object), ("Stream", lambda: stream), ("current_stream", lambda: stream),
+    for name, fake in (("CUDAGraph", object), ("is_current_stream_capturing", lambda: False),
+                       ("Stream", lambda: stream), ("current_stream", lambda: stream),
                        ("stream", lambda s: contextlib.nullcontext()), ("graph", graph)):
         monkeypatch.setattr(torch.cuda, name, fake)
 
@@ -761,3 +762,43 @@ def test_no_collection_falls_into_a_capture(monkeypatch):
     finally:
         gc.set_threshold(*thresholds)
     assert collected == [False] * 5
+
+
+def test_an_update_graph_dropped_in_a_capture_of_the_callers_outlives_it(monkeypatch):
+    """A state's graphs that the collector reaches while the caller captures are
+    destroyed with the next captured update, not there."""
+    import contextlib
+    import gc
+    import sys
+    from types import SimpleNamespace
+    from boonta_amd.algorithms import ppo
+
+    capturing, resource = [], object()
+
+    class Graph:   # holds its resource until its last reference goes, as a HIP graph
+        def __init__(self):
+            self.resource = resource
+
+        def replay(self):
+            pass
+
+    alive = lambda: sys.getrefcount(resource) - none
+    none = sys.getrefcount(resource)
+    stream = SimpleNamespace(cuda_stream=7, wait_stream=lambda s: None)
+    for name, fake in (("CUDAGraph", Graph), ("is_current_stream_capturing", lambda: bool(capturing)),
+                       ("Stream", lambda: stream), ("current_stream", lambda: stream),
+                       ("stream", lambda s: contextlib.nullcontext()),
+                       ("graph", lambda g, stream: contextlib.nullcontext())):
+        monkeypatch.setattr(torch.cuda, name, fake)
+    ex = SimpleNamespace(graphs={(): ppo.capture(lambda st: None)})
+    ex.graphs[()].replay()
+    ex.me = ex
+    del ex
+    capturing.append(1)
+    gc.collect()
+    assert alive() == 1
+    capturing.clear()
+    kept = ppo.capture(lambda st: None)
+    assert alive() == 1
+    del kept
+    assert alive() == 0
