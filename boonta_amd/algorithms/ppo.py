@@ -84,7 +84,7 @@ class UpdateGraph:
     """A captured update.  Its graph outlives it where it is collected while the
     caller captures a graph of their own (a rollout of steps, say, after other
     states were dropped): destroying one there ends the process, so it waits for
-    the next captured update."""
+    the next one captured or destroyed outside."""
 
     _held: list = []
 
@@ -95,8 +95,12 @@ class UpdateGraph:
         self.graph.replay()
 
     def __del__(self):
-        if torch is not None and torch.cuda.is_current_stream_capturing():
-            UpdateGraph._held.append(self.graph)
+        if torch is None:
+            return
+        if torch.cuda.is_current_stream_capturing():
+            self._held.append(self.graph)
+        else:
+            self._held.clear()
 
 
 def capture(issue) -> UpdateGraph:

@@ -3,7 +3,7 @@
  *
  * These are the entry points the XLA FFI custom-call targets of boonta's
  * learner bind (one handler per target, each forwarding XLA's stream and
- * buffers to the launcher below; see INTEGRATION.md).  They take a HIP stream
+ * buffers to the launcher below).  They take a HIP stream
  * as `void*`, device pointers and sizes; enqueue work asynchronously; never
  * synchronise, allocate, or retain pointers across calls; and return 0 or a
  * negative status, with a message from ppo_last_error() on the calling thread.
